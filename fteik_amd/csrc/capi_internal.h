@@ -113,8 +113,17 @@ struct Locator {
     unsigned char *d_skip = nullptr;
     unsigned long long *d_best = nullptr;
     double *d_tmp = nullptr;
+    // per event: it has a pick and its picks are finite (capi_locate.cpp)
+    std::vector<unsigned char> plain;
+    // the origin-time work array (d_t0) still has to take the estimate of
+    // the last event located without it: that event's picks
+    bool t0Stale = false;
+    std::vector<float> t0Obs, t0Wt;
+    std::vector<unsigned char> t0Skip;
 };
 extern Locator gl;
+// The locator's tables changed (their index is out of date).
+void locator_tables_changed();
 
 int padlength32(int alignment, int n);
 float weight_norm(const float *w, int lntf);

@@ -1,6 +1,7 @@
 // capi_locate.cpp -- the travel-time grid-search locator entry points
 // (locate.F90).
 #include "capi_internal.h"
+#include "locate_index.h"
 
 using namespace fteik_capi;
 
@@ -8,6 +9,7 @@ namespace fteik_capi {
 
 static void free_locator()
 {
+    index_release();
     dfree(gl.d_tab); dfree(gl.d_t0); dfree(gl.d_obs); dfree(gl.d_wt);
     dfree(gl.d_xn); dfree(gl.d_skip); dfree(gl.d_best); dfree(gl.d_tmp);
     int rc = gl.refCompat;
@@ -108,6 +110,7 @@ void locate_initialize(int nEvents, int ntf, int ngrd, int *ierr)
     gl.obs.assign((size_t) nEvents*gl.lntf, 0.0f);
     gl.wt.assign((size_t) nEvents*gl.lntf, 0.0f);
     gl.skip.assign((size_t) nEvents*gl.lntf, 1);
+    gl.plain.assign((size_t) nEvents, 0);
     const long nwork = std::max(ngrd, 512);
     if (!dalloc(&gl.d_tab, (size_t) ntf*gl.ldgrd) ||
         !dalloc(&gl.d_t0, nwork) || !dalloc(&gl.d_obs, gl.lntf) ||
@@ -155,6 +158,7 @@ void locate_setTravelTimeField64f(int ngrdIn, int itf, const double *tt,
         return;
     }
     if (!gl.d_tmp && !dalloc(&gl.d_tmp, gl.ngrd)) { *ierr = 1; return; }
+    locator_tables_changed();
     if (!h2d(gl.d_tmp, tt, (size_t) gl.ngrd*sizeof(double)) ||
         fteik_k_tables_d2f(gl.d_tab + (long) (itf - 1)*gl.ldgrd, gl.d_tmp,
                            gl.ngrd, g_dev.stream) || !sync_ok()) *ierr = 1;
@@ -181,6 +185,7 @@ void locate_setTravelTimeField32f(int ngrdIn, int itf, const float *tt,
         *ierr = 1;
         return;
     }
+    locator_tables_changed();
     if (!h2d(gl.d_tab + (long) (itf - 1)*gl.ldgrd, tt,
              (size_t) gl.ngrd*sizeof(float))) *ierr = 1;
 }
@@ -234,14 +239,19 @@ void locate_setObservation64f(int evnmbr, int nttimes, bool lhaveOT,
     for (int i = 0; i < gl.lntf; i++) {
         gl.obs[k + i] = 0.0f; gl.wt[k + i] = 0.0f; gl.skip[k + i] = 1;
     }
+    bool any = false, plain = true;
     for (int i = 0; i < nttimes; i++) {
         const size_t j = k + (size_t) (obs2tf[i] - 1);
         if (wts[i] > 0.0) {
             gl.obs[j] = (float) (picks[i] - tmax);
             gl.wt[j] = (float) wts[i];
             gl.skip[j] = 0;
+            any = true;
+            plain = plain && fabsf(gl.obs[j]) <= kPlainLimit &&
+                    gl.wt[j] <= kPlainLimit && gl.wt[j] >= 1.0f/kPlainLimit;
         }
     }
+    gl.plain[(size_t) (evnmbr - 1)] = any && plain;
 }
 
 void locate_setObservation64fC(const int evnmbr, const int nttimes,
@@ -279,8 +289,38 @@ void locate_locateEvent(int evnmbr, int *optIndx, double *t0Opt,
         return;
     }
     const size_t k = (size_t) (evnmbr - 1)*gl.lntf;
+    if (!gl.refCompat) {
+        const int rc = index_search(1, &evnmbr, optIndx, t0Opt, objOpt);
+        if (rc == 0) {
+            // the work array takes this event's estimate when it is next
+            // read
+            gl.t0Stale = true;
+            gl.t0Obs.assign(&gl.obs[k], &gl.obs[k] + gl.lntf);
+            gl.t0Wt.assign(&gl.wt[k], &gl.wt[k] + gl.lntf);
+            gl.t0Skip.assign(&gl.skip[k], &gl.skip[k] + gl.lntf);
+            return;
+        }
+        if (rc == 2) {
+            msg("locate_locateEvent: GPU error");
+            return;
+        }
+    }
     const float xnorm = weight_norm(gl.wt.data() + k, gl.lntf);
     const unsigned long long init = ~0ull;
+    if (gl.t0Stale && gl.refCompat) {
+        if (!h2d(gl.d_obs, gl.t0Obs.data(), gl.lntf*sizeof(float)) ||
+            !h2d(gl.d_wt, gl.t0Wt.data(), gl.lntf*sizeof(float)) ||
+            !h2d(gl.d_skip, gl.t0Skip.data(), (size_t) gl.lntf) ||
+            !h2d(gl.d_best, &init, sizeof(init)) ||
+            fteik_k_locate(gl.d_tab, gl.ntf, gl.ngrd, gl.ldgrd, gl.d_obs,
+                           gl.d_wt, gl.d_skip, gl.lntf,
+                           weight_norm(gl.t0Wt.data(), gl.lntf), gl.d_t0,
+                           nullptr, 0, gl.d_best, g_dev.stream) != 0) {
+            msg("locate_locateEvent: GPU error");
+            return;
+        }
+    }
+    gl.t0Stale = false;
     bool ok = h2d(gl.d_obs, gl.obs.data() + k, gl.lntf*sizeof(float)) &&
               h2d(gl.d_wt, gl.wt.data() + k, gl.lntf*sizeof(float)) &&
               h2d(gl.d_skip, gl.skip.data() + k, (size_t) gl.lntf) &&
@@ -332,6 +372,11 @@ void locate_locateEvents(int n, const int *evnmbr, int *optIndx,
             *ierr = 1;
             return;
         }
+    {
+        const int rc = index_search(n, evnmbr, optIndx, t0Opt, objOpt);
+        if (rc == 2) { msg("locate_locateEvents: GPU error"); *ierr = 1; }
+        if (rc != 1) return;
+    }
     std::vector<float> o((size_t) n*gl.lntf), w((size_t) n*gl.lntf), xn((size_t) n);
     std::vector<unsigned char> sk((size_t) n*gl.lntf);
     for (int e = 0; e < n; e++) {

@@ -57,6 +57,34 @@ struct BatchGrid {
     int nz, nx, ny, zsi, xsi, ysi;
 };
 
+// Index of the locator's tables (locate_index.hip; device pointers).  The
+// ngrd cells are taken as an nz x nx x ny grid (z fastest) cut into blocks
+// of 2^lz x 2^lx x 2^ly = 64 cells, the blocks into groups of as many.
+struct LocIndex {
+    int nz, nx, ny, lz, lx, ly;
+    int nbz, nbx, nby, nb;         // blocks
+    int nsz, nsx, nsy, ns;         // groups
+    int ntf, nt;                   // tables; padded (fteik_k_locate_index_nt)
+    float* perm;                   // [nb][ntf][64] times in block order
+    float *rep, *h;                // [ntf][nb] representative, difference
+    float *srep, *sh;              // [ntf][ns] the groups'
+    unsigned* tmax;                // largest |time| (bits; inf: not finite)
+    // search work space for eb events at a time
+    int eb;
+    float* lbs;                    // [ns][eb] bounds of the groups
+    int* pair;                     // [ns*eb][2] (group, event) that stay
+    int* npair;                    // their count (8 bytes)
+    float* lbc;                    // [ns*eb][64] bounds of their blocks
+};
+constexpr int kLocEv = 8;          // events per group of picks
+struct LocEvents {
+    float *o8, *w8, *h8;           // [n/8][ntf][8] picks, w, sqrt(1/2) w
+    float* row;                    // [n][nt][3] the same by event
+    float *xn, *kap, *mar;         // [n] 1/sum w, kappa, rounding margin
+    unsigned long long* best;      // [n] argmin keys
+    float* t0;                     // [n] origin times
+};
+
 // Grid of a ray trace (rays.hip): 2D grids have ny = 1 and is3d = 0.
 struct RayGrid {
     int is3d, nz, nx, ny;
@@ -191,6 +219,23 @@ int fteik_k_statics(float* tstatic, const float* tobs, const float* tt,
                     const float* wts, const float* t0, int ldo, int nobs,
                     int nev, hipStream_t stream);
 // locate.hip (continued)
+// locate_index.hip
+int fteik_k_locate_index_nt(int ntf);    // 0: too many tables for an index
+int fteik_k_locate_strides(const float* tab, long ldgrd, int ntf, int ngrd,
+                           const int* p, int np, float* d, hipStream_t s);
+int fteik_k_locate_index_build(const fteik::LocIndex* g, const float* tab,
+                               long ldgrd, hipStream_t s);
+int fteik_k_locate_index_events(const fteik::LocIndex* g,
+                                const fteik::LocEvents* v, int n, int lntf,
+                                const float* obs, const float* wt,
+                                const unsigned char* skip, hipStream_t s);
+int fteik_k_locate_index_search(const fteik::LocIndex* g,
+                                const fteik::LocEvents* v, int e0, int n,
+                                int ncu, hipStream_t s);
+int fteik_k_locate_index_origin(const fteik::LocIndex* g,
+                                const fteik::LocEvents* v, int n,
+                                const float* tab, long ldgrd, int lntf,
+                                const unsigned char* skip, hipStream_t s);
 int fteik_k_locate_t0_at(float* t0, const float* tables, int ntf, long ldgrd,
                          const float* obs, const float* wt,
                          const unsigned char* skip, const float* xnorm,
