@@ -20,7 +20,7 @@ LIB = os.path.join(LIBDIR, "libfteik_shared.so")
 SOURCES = ["capi_common.cpp", "capi3d.cpp", "capi2d.cpp", "capi_locate.cpp",
            "capi_model.cpp", "capi_batch.cpp", "capi_surrogate.cpp",
            "capi_rays.cpp", "capi_locate_index.cpp", "locate_noalloc.hip",
-           "sweep3d.hip", "sweep2d.hip", "util.hip", "locate.hip", "locate_index.hip",
+           "sweep3d.hip", "sweep_chunk.hip", "sweep2d.hip", "util.hip", "locate.hip", "locate_index.hip",
            "stencil_eval.hip", "batch3d.hip", "surrogate.hip", "rays.hip"]
 
 # -ffp-contract=off: no FMA contraction, so the FP64 path keeps the

@@ -14,7 +14,7 @@
 // waits on lower ids, which were dispatched before it on their own XCD and
 // are running or done.  Every wait keeps the spin limit of the body.
 #include <hip/hip_runtime.h>
-#include "sweep_pencil.h"
+#include "sweep_chunk.h"
 
 namespace fteik {
 
@@ -51,6 +51,8 @@ void batch_sweep_kernel(const BatchGrid* __restrict__ grids,
     a.mb = nullptr;
     a.mbx = a.mby = nullptr; a.mbnt = 0;
     a.colmod = nullptr; a.plan = nullptr;
+    a.stamp = nullptr; a.lastchg = nullptr;
+    a.count = 0; a.code = 0; a.mbBytes = 0;
     if (a.fz0 > a.fz1 || a.fx0 > a.fx1 || a.fy0 > a.fy1) {
         if (threadIdx.x == 0)
             __hip_atomic_store(flags + m.flag, (serial << 32) | 0xffffffffull,
@@ -94,7 +96,7 @@ __global__ void batch_mb_args_kernel(const BatchGrid* __restrict__ grids,
                                      int bx, int by,
                                      unsigned long long serial,
                                      int* __restrict__ err, int fp32,
-                                     int track,
+                                     int track, unsigned count,
                                      SweepArgs<R>* __restrict__ args)
 {
     const int i = blockIdx.x*blockDim.x + threadIdx.x;
@@ -120,6 +122,10 @@ __global__ void batch_mb_args_kernel(const BatchGrid* __restrict__ grids,
     a.mbx = g.mbx; a.mby = g.mby; a.mbnt = g.mbnt;
     a.colmod = nullptr; a.plan = nullptr; a.prog = nullptr;
     a.pserial = 0; a.par = 0; a.psz = a.psx = a.psy = 0;
+    a.stamp = count ? g.stamp : nullptr;
+    a.lastchg = g.lastchg;
+    a.count = count; a.code = stamp_code(count);
+    a.mbBytes = g.mbBytes;
     args[i] = a;
 }
 
@@ -284,13 +290,21 @@ extern "C" int fteik_k_batch_mb_sweep(const BatchGrid* grids, int ngrids,
                                       int sweep, int linit,
                                       unsigned long long serial,
                                       int* err, int fp32, int track,
+                                      int chunk, unsigned count, int cube,
                                       void* argbuf, hipStream_t stream)
 {
     if (tile < 0 || tile >= kNumTiles || kTiles[tile].mode == 0 || nwg < 0 ||
         ngrids < 1 || sweep < 1 || sweep > 8 || !argbuf) return 2;
     if (nwg == 0) return 0;                 // every grid's box is empty
     const TileShape ts = kTiles[tile];
-    const void* fn = linit
+    // chunked tiles (iteration sweeps only): the map of an 8 x 8 tile
+    if (linit) chunk = 0;
+    if (chunk && (ts.bx != CB || ts.by != CB)) return 2;
+    // count: number of the iteration sweep in the record, 0 without one
+    if (!chunk) count = 0;
+    const void* fn = chunk
+        ? fteik_k_chunk_fn(fp32, count, cube)
+        : linit
         ? (fp32 ? batch_mb_fn<float, true>(tile)
                 : batch_mb_fn<double, true>(tile))
         : (fp32 ? batch_mb_fn<float, false>(tile)
@@ -298,16 +312,17 @@ extern "C" int fteik_k_batch_mb_sweep(const BatchGrid* grids, int ngrids,
     if (fp32)
         hipLaunchKernelGGL(batch_mb_args_kernel<float>, dim3((ngrids + 63)/64),
                            dim3(64), 0, stream, grids, ngrids, sweep, linit,
-                           ts.bx, ts.by, serial, err, fp32, track,
+                           ts.bx, ts.by, serial, err, fp32, track, count,
                            (SweepArgs<float>*) argbuf);
     else
         hipLaunchKernelGGL(batch_mb_args_kernel<double>,
                            dim3((ngrids + 63)/64), dim3(64), 0, stream, grids,
                            ngrids, sweep, linit, ts.bx, ts.by, serial, err,
-                           fp32, track, (SweepArgs<double>*) argbuf);
+                           fp32, track, count,
+                           (SweepArgs<double>*) argbuf);
     void* args[] = {&argbuf, (void*) &map};
     hipError_t e = hipLaunchKernel(fn, dim3(nwg),
-                                   dim3(ts.bx*ts.by + 64*ts.mode), args, 0,
-                                   stream);
+                                   dim3(chunk ? 64 : ts.bx*ts.by + 64*ts.mode),
+                                   args, 0, stream);
     return e == hipSuccess ? 0 : 1;
 }

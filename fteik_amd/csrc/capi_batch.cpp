@@ -36,6 +36,11 @@ struct Batch3D {
     // 70 ms against 78 ms for 16 x 16 tiles and 113 ms for the best flag
     // tile on 64 grids of 64..192 per axis)
     int mbTile = 12, mapMbTile = -1;
+    // until a tile shape is chosen, the iteration sweeps run on chunked
+    // tiles where every grid can use them (chunked): 64 grids of 20 .. 160
+    // per axis, converged, 98 -> 29 ms; 8 station tables of 129 x 129 x 65,
+    // 50 -> 31 ms
+    bool chunk = true, chunked = false, mapChunk = false;
     int mbOff[9] = {0}, mbN[9] = {0};
     unsigned long long *d_mb = nullptr;
     size_t mbCap = 0;
@@ -44,6 +49,13 @@ struct Batch3D {
     size_t mbeCap = 0;
     int *d_mbmap = nullptr;
     char *d_mbargs = nullptr;
+    // change record of the chunked tiles' iteration sweeps: the grids' bytes
+    // one after another, then a word per grid (last changing sweep); count:
+    // sweeps recorded
+    unsigned char *d_stamp = nullptr;
+    size_t stampCap = 0;
+    unsigned count = 0;
+    bool cube = false;               // every grid has equal spacings
     int *d_err = nullptr;
     double *d_maxdelta = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -60,7 +72,7 @@ void free_batch()
     }
     dfree(gb.d_desc); dfree(gb.d_map); dfree(gb.d_flags); dfree(gb.d_err);
     dfree(gb.d_maxdelta); dfree(gb.d_mb); dfree(gb.d_mbmap); dfree(gb.d_mbe);
-    dfree(gb.d_mbargs);
+    dfree(gb.d_mbargs); dfree(gb.d_stamp);
     if (gb.ev0) hipEventDestroy(gb.ev0);
     if (gb.ev1) hipEventDestroy(gb.ev1);
     gb = Batch3D();
@@ -117,6 +129,36 @@ bool batch_prepare(const char *who)
                            g_dev.stream);
         }
     }
+    gb.chunked = gb.chunk && edge;
+    for (const BGrid &x : gb.g)
+        gb.chunked = gb.chunked && fteik_k_chunk_fits(
+            x.nz, x.nx, x.ny, sizeof(unsigned long long)*
+            (edge_words(x, false) + edge_words(x, true)));
+    // change record (chunked tiles): words first, then each grid's bytes;
+    // where it finds no memory the streamed tiles run every sweep
+    size_t stoff = ((size_t) ng*sizeof(unsigned) + 255)/256*256;
+    if (gb.chunked) {
+        size_t bytes = stoff;
+        for (const BGrid &x : gb.g)
+            bytes += fteik_k_stamp_bytes((long) x.nz*x.nx*x.ny);
+        if (bytes > gb.stampCap) {
+            dfree(gb.d_stamp);
+            gb.stampCap = 0;
+            if (dalloc(&gb.d_stamp, bytes)) {
+                gb.stampCap = bytes;
+            } else {
+                hipGetLastError();
+                gb.chunked = false;
+            }
+        }
+    }
+    if (!gb.chunked) {
+        dfree(gb.d_stamp);
+        gb.stampCap = 0;
+    }
+    gb.cube = true;
+    for (const BGrid &x : gb.g)
+        gb.cube = gb.cube && x.dz == x.dx && x.dz == x.dy;
     size_t mboff = 0, mbeoff = 0;
     for (int i = 0; i < ng; i++) {
         const BGrid &x = gb.g[(size_t) i];
@@ -127,12 +169,23 @@ bool batch_prepare(const char *who)
         d.mb = gb.mbTile >= 0 ? gb.d_mb + mboff : nullptr;
         mboff += 2*(size_t) x.nz*x.nx*x.ny;
         d.mbx = d.mby = nullptr;
+        d.mbBytes = 0;
         d.mbnt = x.nz + x.nx + x.ny;
         if (edge) {
             d.mbx = gb.d_mbe + mbeoff;
             mbeoff += edge_words(x, false);
             d.mby = gb.d_mbe + mbeoff;
             mbeoff += edge_words(x, true);
+            d.mbBytes = (unsigned) (sizeof(unsigned long long)*
+                                    (edge_words(x, false) +
+                                     edge_words(x, true)));
+        }
+        d.stamp = nullptr;
+        d.lastchg = nullptr;
+        if (gb.d_stamp) {
+            d.stamp = gb.d_stamp + stoff + fteik_k_stamp_offset();
+            d.lastchg = (unsigned *) gb.d_stamp + i;
+            stoff += fteik_k_stamp_bytes((long) x.nz*x.nx*x.ny);
         }
         d.nz = x.nz; d.nx = x.nx; d.ny = x.ny;
         d.zsi = x.src.zsi; d.xsi = x.src.xsi; d.ysi = x.src.ysi;
@@ -200,6 +253,7 @@ bool batch_prepare(const char *who)
         }
     }
     gb.mapMbTile = gb.mbTile;
+    gb.mapChunk = gb.chunk;
     return true;
 }
 
@@ -213,6 +267,10 @@ bool batch_sweep(int sweep, bool linit, bool fp32, bool track)
                                               gb.mbTile, sweep, linit ? 1 : 0,
                                               ++gb.serial, gb.d_err,
                                               fp32 ? 1 : 0, track ? 1 : 0,
+                                              gb.chunked ? 1 : 0,
+                                              (!linit && gb.chunked)
+                                              ? ++gb.count : 0,
+                                              gb.cube ? 1 : 0,
                                               gb.d_mbargs, g_dev.stream);
         if (rc != 0) msg("fteik_batch3d_solve: sweep launch failed (%d)", rc);
         return rc == 0;
@@ -223,6 +281,14 @@ bool batch_sweep(int sweep, bool linit, bool fp32, bool track)
                                  g_dev.stream);
     if (rc != 0) msg("fteik_batch3d_solve: sweep launch failed (%d)", rc);
     return rc == 0;
+}
+
+// Starts a new change record.
+bool batch_reset_record()
+{
+    gb.count = 0;
+    return !gb.chunked || hipMemsetAsync(gb.d_stamp, 0, gb.stampCap,
+                                         g_dev.stream) == hipSuccess;
 }
 
 double batch_updates_init()
@@ -382,6 +448,7 @@ void fteik_batch3d_setTile(int tile, int *ierr)
     }
     // a flag tile (mode 0) or a mailbox tile (modes 1, 2) serves every
     // sweep
+    gb.chunk = false;
     if (fteik_k_tile_mode(tile) == 0) {
         gb.tile = tile;
         gb.mbTile = -1;
@@ -432,7 +499,8 @@ void fteik_batch3d_solve(int nsweep, double eps, int *ierr)
         }
         gb.mapTile = -1;
     }
-    if ((gb.mapTile != gb.tile || gb.mapMbTile != gb.mbTile) &&
+    if ((gb.mapTile != gb.tile || gb.mapMbTile != gb.mbTile ||
+         gb.mapChunk != gb.chunk) &&
         !batch_prepare(who)) { *ierr = 1; return; }
     hipMemsetAsync(gb.d_err, 0, sizeof(int), g_dev.stream);
     bool ok = true;
@@ -441,6 +509,7 @@ void fteik_batch3d_solve(int nsweep, double eps, int *ierr)
     int corr = 0;
     bool converged = true;
     if (gb.precision == 0) {
+        ok = ok && batch_reset_record();
         for (int k = 0; k < nsweep && ok; k++)
             for (int sw = 1; sw <= 8 && ok; sw++)
                 ok = batch_sweep(sw, false, false, false);
@@ -454,6 +523,7 @@ void fteik_batch3d_solve(int nsweep, double eps, int *ierr)
                     && fteik_k_consts_to_float(x.d_cst, x.d_cst32,
                                                g_dev.stream) == 0;
         }
+        ok = ok && batch_reset_record();
         for (int k = 0; k < nsweep && ok; k++)
             for (int sw = 1; sw <= 8 && ok; sw++)
                 ok = batch_sweep(sw, false, true, false);
@@ -465,6 +535,7 @@ void fteik_batch3d_solve(int nsweep, double eps, int *ierr)
         const size_t ng = gb.g.size();
         std::vector<double> md(ng);
         converged = false;
+        ok = ok && batch_reset_record();
         for (corr = 0; corr < gb.maxCorr && ok; ) {
             hipMemsetAsync(gb.d_maxdelta, 0, ng*sizeof(double), g_dev.stream);
             for (int sw = 1; sw <= 8 && ok; sw++)
@@ -507,6 +578,7 @@ void fteik_batch3d_autotune(int nsweep, double eps, int *tile, int *ierr)
     if (!gb.init) { msg("%s: batch not initialized", who); *ierr = 1;
                     return; }
     const int keepTile = gb.tile, keepMb = gb.mbTile;
+    const bool keepChunk = gb.chunk;
     int best = -1;
     double bestMs = 0.0;
     for (int t = 0; t < fteik_k_num_tiles(); t++) {
@@ -519,10 +591,18 @@ void fteik_batch3d_autotune(int nsweep, double eps, int *tile, int *ierr)
     }
     gb.tile = keepTile;
     gb.mbTile = keepMb;
+    gb.chunk = keepChunk;
     if (best < 0) { msg("%s: no tile shape solved the batch", who);
                     *ierr = 1; return; }
     int e = 0;
-    fteik_batch3d_setTile(best, &e);
+    // chunked tiles, their initialization sweeps on the default shape
+    gb.mbTile = Batch3D().mbTile;
+    gb.chunk = true;
+    fteik_batch3d_solve(nsweep, eps, &e);
+    if (e == 1 || !gb.chunked || gb.last_ms >= bestMs)
+        fteik_batch3d_setTile(best, &e);
+    else
+        best = gb.mbTile;
     fteik_batch3d_solve(nsweep, eps, &e);
     if (e == 1) { *ierr = 1; return; }
     *tile = best;

@@ -55,6 +55,9 @@ struct BatchGrid {
     unsigned long long* mby;       // per-node one), as SweepLaunch::mbx/mby
     int mbnt;
     int nz, nx, ny, zsi, xsi, ysi;
+    unsigned char* stamp;          // chunked tiles' change record
+    unsigned* lastchg;
+    unsigned mbBytes;
 };
 
 // Index of the locator's tables (locate_index.hip; device pointers).  The
@@ -119,8 +122,16 @@ size_t fteik_k_batch_mb_args_bytes(int ngrids);
 int fteik_k_batch_mb_sweep(const fteik::BatchGrid* grids, int ngrids,
                            const int* map, int nwg, int tile, int sweep,
                            int linit, unsigned long long serial, int* err,
-                           int fp32, int track, void* argbuf,
-                           hipStream_t stream);
+                           int fp32, int track, int chunk, unsigned count,
+                           int cube, void* argbuf, hipStream_t stream);
+// sweep_chunk.hip: the chunked tiles' kernels (count: number of the sweep
+// in the record, 0 without one; cube: every grid has equal spacings),
+// whether a grid can use them (mbBytes: of its edge-major mailboxes), the
+// bytes of its change record
+int fteik_k_chunk_fits(int nz, int nx, int ny, size_t mbBytes);
+const void* fteik_k_chunk_fn(int fp32, unsigned count, int cube);
+size_t fteik_k_stamp_bytes(long ngrd);
+long fteik_k_stamp_offset(void);
 // sweep3d.hip
 int fteik_k_sweep3d(const fteik::SweepLaunch* L, int sweep, int linit,
                     hipStream_t stream);

@@ -42,6 +42,8 @@ __device__ __forceinline__ double rmin(double a, double b) { return __builtin_fm
 __device__ __forceinline__ double rmax(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ float rmin(float a, float b) { return __builtin_fminf(a, b); }
 __device__ __forceinline__ float rmax(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ double rabs(double a) { return __builtin_fabs(a); }
+__device__ __forceinline__ float rabs(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ double rsqrt_exact(double x) { return __builtin_sqrt(x); }
 __device__ __forceinline__ float rsqrt_exact(float x) { return __builtin_sqrtf(x); }
 
@@ -95,6 +97,26 @@ __device__ __forceinline__ double sqrt_pos(double x)
 }
 __device__ __forceinline__ float sqrt_pos(float x) { return __builtin_sqrtf(x); }
 
+// As sqrt_pos, and 0 for 0: the estimate is taken of an argument raised to
+// at least 2^-800, whose estimate times 0 is 0 and stays 0.  The 3D
+// operator's argument t2 - t3, where its gate t2 >= t3 is open, is 0 or at
+// least an ulp of t2 = 9 s^2 (1/dz^2 + 1/dx^2 + 1/dy^2) >= 2^-395
+// (velocities and spacings are at most 1e30), so never below 2^-767.
+__device__ __forceinline__ double sqrt_nonneg(double x)
+{
+    const double y = __builtin_amdgcn_rsq(lmax(x, 0x1p-800));
+    double g = x*y;
+    double h = y*0.5;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    return __builtin_fma(d, h, g);
+}
+__device__ __forceinline__ float sqrt_nonneg(float x) { return __builtin_sqrtf(x); }
+
 // localSolver.F90:775-792
 template <typename R>
 __device__ __forceinline__ R tana3d(int i, int j, int k, const Consts<R>& c)
@@ -142,8 +164,9 @@ struct Slw { R s1, s2, s3, s4, s5, s6, s7; };
 // so the compiler can interleave them instead of branching around each.
 // Where a gate is closed the value computed under it is discarded (it may
 // be NaN); where it is open the value is computed in the reference's
-// operation order, so results are bitwise those of the gated form.
-template <typename R>
+// operation order, so results are bitwise those of the gated form.  CUBE:
+// equal spacings, where a 2D gate's two bounds are one.
+template <typename R, bool CUBE = false>
 __device__ __forceinline__ R noinit3d(const Consts<R>& c, const Nbr<R>& t,
                                       const Slw<R>& s, R tupd_in)
 {
@@ -165,7 +188,8 @@ __device__ __forceinline__ R noinit3d(const Consts<R>& c, const Nbr<R>& t,
               + sqrt_pos(four_sref2*c.dz2i_p_dx2i - c.dz2i_dx2i*tab2))
               *c.dz2i_p_dx2i_inv;
     }
-    const bool g1 = temtv < c.dz*s.s4 && -temtv < c.dx*s.s4;
+    const bool g1 = CUBE ? rabs(temtv) < c.dz*s.s4
+                         : temtv < c.dz*s.s4 && -temtv < c.dx*s.s4;
     // ZY plane
     const R tvmtn = t.tv - t.tn;
     R t2_2d;
@@ -180,7 +204,8 @@ __device__ __forceinline__ R noinit3d(const Consts<R>& c, const Nbr<R>& t,
               + sqrt_pos(four_sref2*c.dz2i_p_dy2i - c.dz2i_dy2i*tab2))
               *c.dz2i_p_dy2i_inv;
     }
-    const bool g2 = tvmtn < c.dy*s.s5 && -tvmtn < c.dz*s.s5;
+    const bool g2 = CUBE ? rabs(tvmtn) < c.dz*s.s5
+                         : tvmtn < c.dy*s.s5 && -tvmtn < c.dz*s.s5;
     // XY plane
     const R temtn = t.te - t.tn;
     R t3_2d;
@@ -195,7 +220,8 @@ __device__ __forceinline__ R noinit3d(const Consts<R>& c, const Nbr<R>& t,
               + sqrt_pos(four_sref2*c.dx2i_p_dy2i - c.dx2i_dy2i*tab2))
               *c.dx2i_p_dy2i_inv;
     }
-    const bool g3 = temtn < c.dy*s.s6 && -temtn < c.dx*s.s6;
+    const bool g3 = CUBE ? rabs(temtn) < c.dz*s.s6
+                         : temtn < c.dy*s.s6 && -temtn < c.dx*s.s6;
     // 3D operator
     R t3d_v, t2, t3;
     {
@@ -212,7 +238,7 @@ __device__ __forceinline__ R noinit3d(const Consts<R>& c, const Nbr<R>& t,
         const R tac2 = tac*tac;
         t3 = c.dz2dx2*tab2 + c.dz2dy2*tbc2 + c.dx2dy2*tac2;
         const R t1 = tb*c.dz2i + ta*c.dx2i + tc*c.dy2i;
-        t3d_v = (t1 + rsqrt_exact(t2 - t3))*c.dsumi;
+        t3d_v = (t1 + sqrt_nonneg(t2 - t3))*c.dsumi;
     }
     // the reference's order of minimisation
     t12min = rmin(t12min, g1 ? t1_2d : huge);

@@ -1,0 +1,63 @@
+// sweep_chunk.hip -- the batch's kernels of the chunked tile
+// (sweep_chunk.h).  No launch is cooperative: a tile waits only on tiles of
+// lower-numbered workgroups and workgroups are dispatched in order, so the
+// lowest unfinished tile is always resident and every wait ends; each wait
+// also has a spin limit that turns a hang into a reported error.
+#include <hip/hip_runtime.h>
+#include "sweep_chunk.h"
+
+namespace fteik {
+
+// Workgroup w sweeps map entry (grid, tile); args[g]: grid g's sweep
+// arguments for this launch, read through the constant address space as in
+// batch_mb_kernel.
+template <typename R, bool SKIP, bool RECORD, bool CUBE>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(3)))
+void batch_chunk_kernel(const SweepArgs<R>* __restrict__ args,
+                        const int* __restrict__ map)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef const __attribute__((address_space(4))) SweepArgs<R> CArgs;
+    const SweepArgs<R> a = ((CArgs*) args)[map[2*blockIdx.x]];
+#else   // the host pass only parses the kernel
+    const SweepArgs<R> a = args[map[2*blockIdx.x]];
+#endif
+    chunk_body<R, SKIP, RECORD, CUBE>(a, map[2*blockIdx.x + 1]);
+}
+
+// kind 0: every chunk; 1: every chunk, changes recorded; 2: skipping
+template <typename R, bool CUBE>
+static const void* chunk_fn(int kind)
+{
+#define CF(f) (kind == 0 ? (const void*) f<R, false, false, CUBE> \
+               : kind == 1 ? (const void*) f<R, false, true, CUBE> \
+                           : (const void*) f<R, true, true, CUBE>)
+    return CF(batch_chunk_kernel);
+#undef CF
+}
+
+} // namespace fteik
+
+using namespace fteik;
+
+extern "C" const void* fteik_k_chunk_fn(int fp32, unsigned count, int cube)
+{
+    const int kind = count == 0 ? 0 : count <= 8 ? 1 : 2;
+    if (fp32) return cube ? chunk_fn<float, true>(kind)
+                          : chunk_fn<float, false>(kind);
+    return cube ? chunk_fn<double, true>(kind)
+                : chunk_fn<double, false>(kind);
+}
+
+extern "C" int fteik_k_chunk_fits(int nz, int nx, int ny, size_t mbBytes)
+{
+    return chunk_fits(nz, nx, ny, mbBytes) ? 1 : 0;
+}
+
+extern "C" size_t fteik_k_stamp_bytes(long ngrd)
+{
+    return (size_t) ngrd + 2*kStampPad;
+}
+
+extern "C" long fteik_k_stamp_offset(void) { return kStampPad; }

@@ -160,6 +160,16 @@ struct SweepArgs {
     unsigned long long pserial;
     int par;
     int psz, psx, psy;
+    // Chunked tiles with skipping (sweep_chunk.h; null: off):
+    //   stamp[node]   number (stamp_code) of the sweep that changed it last
+    //   lastchg       number of the last sweep that changed anything
+    //   count, code   number of this sweep (1: the solve's first iteration
+    //                 sweep) and its stamp code
+    unsigned char* stamp;
+    unsigned* lastchg;
+    unsigned count;
+    int code;
+    unsigned mbBytes;            // of mbx and, after it, mby
 };
 
 // The per-sweep values of a mailbox sweep, kept apart from SweepArgs so a

@@ -301,11 +301,16 @@ void fteik_batch3d_setPrecision(int mode, int *ierr);
 void fteik_batch3d_setMixedParameters(double bias, int maxCorrections,
                                       int *ierr);
 /* tile shape of the batch (see fteik_solver3d_setTile), flag (mode 0) or
- * mailbox (modes 1, 2); it serves every sweep (default: mailbox tile 12) */
+ * mailbox (modes 1, 2); it serves every sweep.  Until one is chosen the
+ * initialization sweeps run on mailbox tile 12 and the iterations on chunked
+ * 8 x 8 tiles, which skip nodes that cannot change (grids too large for
+ * 32-bit offsets, or no memory for their change record: tile 12) */
 void fteik_batch3d_setTile(int tile, int *ierr);
 /* EXTENSION: the batch autotuner: times fteik_batch3d_solve(nsweep, eps)
  * with every tile shape (flag and mailbox tiles), keeps the fastest and
- * returns it; the batch is left solved with it. */
+ * returns it; the batch is left solved with it.  If the chunked tiles are
+ * faster than every shape the batch is left with them and tile is 12, the
+ * shape of their initialization sweeps. */
 void fteik_batch3d_autotune(int nsweep, double eps, int *tile, int *ierr);
 void fteik_batch3d_solve(int nsweep, double eps, int *ierr);
 void fteik_batch3d_getLastSolveInfo(double *ms, int *corrIterations,

@@ -1,0 +1,83 @@
+"""The chunked tiles of a batch's iteration sweeps (the default until a tile
+shape is chosen): fields equal the oracle's bit for bit, and the streamed tiles'
+where the oracle has no such mode, at the edges of tiles (8 x 8 columns),
+chunks (4 levels) and runs (4,092 levels), with and without skipping."""
+from ctypes import byref, c_int
+
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from tests.gpu_helpers import lib, _d
+
+pytestmark = pytest.mark.gpu
+
+# nz, nx, ny, (dz, dx, dy), source in cells, iterations.  Random velocities
+# in every cell bend the rays, so fields keep changing for several iterations
+# in ever fewer places.
+CASES = [
+    (3, 3, 3, (10.0, 10.0, 10.0), (0.4, 0.9, 0.7), 3),
+    (4, 9, 10, (10.0, 10.0, 10.0), (1.5, 0.0, 7.9), 4),
+    (5, 17, 8, (10.0, 12.0, 9.0), (0.0, 14.5, 3.2), 6),
+    (18, 16, 25, (5.0, 5.0, 5.0), (15.9, 7.9, 0.1), 9),
+    (33, 41, 34, (10.0, 10.0, 10.0), (16.3, 20.0, 31.7), 12),
+    (61, 26, 33, (7.0, 11.0, 13.0), (3.3, 23.9, 0.0), 12),
+    (4080, 9, 17, (10.0, 10.0, 10.0), (2000.5, 3.0, 8.0), 4),
+    (4100, 9, 17, (10.0, 10.0, 10.0), (4000.0, 0.0, 14.9), 4),
+]
+
+
+def _model(nz, nx, ny, seed):
+    rng = np.random.default_rng(seed)
+    return 1000.0 * rng.uniform(1.0, 6.0, (nz - 1) * (nx - 1) * (ny - 1))
+
+
+def _oracle(vel, nz, nx, ny, d, src, nsweep):
+    slow = orc.cell_slowness(vel, nz, nx, ny, order=0)
+    s = orc.source_locate((nz, nx, ny) + d + (0.0, 0.0, 0.0), *src, slow)
+    return orc.solve3d(slow, nz, nx, ny, *d, s, nsweep, 3.0, schedule=1)
+
+
+@pytest.mark.parametrize("cube", [True, False])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_chunked_batch(cube, precision):
+    """Uneven grids: FP64 against the oracle, mixed against the streamed
+    tiles; solved twice, the second time with the tile shape chosen."""
+    cases = [c[:3] + ((10.0, 10.0, 10.0) if cube else c[3],) + c[4:5]
+             for c in CASES[:7]]
+    nsweep = 9
+    print("case: chunked batch", cube, precision, flush=True)
+    L, ierr = lib(), c_int(1)
+    L.fteik_batch3d_initialize(len(cases), byref(ierr))
+    assert ierr.value == 0
+    models = [_model(*c[:3], 300 + i) for i, c in enumerate(cases)]
+    srcs = [tuple(a * b for a, b in zip(c[4], c[3])) for c in cases]
+    for i, c in enumerate(cases):
+        L.fteik_batch3d_setGrid(i + 1, *c[:3], 0.0, 0.0, 0.0, *c[3],
+                                _d(models[i]), *srcs[i], byref(ierr))
+        assert ierr.value == 0
+    L.fteik_batch3d_setPrecision(precision, byref(ierr))
+    fields, status = [], []
+    for tile in (None, 12):
+        if tile is not None:
+            L.fteik_batch3d_setTile(tile, byref(ierr))
+            assert ierr.value == 0
+        L.fteik_batch3d_solve(nsweep, 3.0, byref(ierr))
+        # 2: corrections of a mixed solve that ran out before it converged
+        assert ierr.value in ((0, 2) if precision else (0,))
+        status.append(ierr.value)
+        got = []
+        for i, c in enumerate(cases):
+            tt = np.zeros(c[0] * c[1] * c[2])
+            L.fteik_batch3d_getTravelTimeField64f(i + 1, tt.size, 0, _d(tt),
+                                                  byref(ierr))
+            assert ierr.value == 0
+            got.append(tt)
+        fields.append(got)
+    L.fteik_batch3d_free()
+    assert status[0] == status[1]
+    for i, c in enumerate(cases):
+        np.testing.assert_array_equal(fields[0][i], fields[1][i])
+        if precision == 0:
+            np.testing.assert_array_equal(
+                fields[0][i], _oracle(models[i], *c[:4], srcs[i], nsweep))
