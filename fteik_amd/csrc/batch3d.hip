@@ -52,7 +52,7 @@ void batch_sweep_kernel(const BatchGrid* __restrict__ grids,
     a.mbx = a.mby = nullptr; a.mbnt = 0;
     a.colmod = nullptr; a.plan = nullptr;
     a.stamp = nullptr; a.lastchg = nullptr;
-    a.count = 0; a.code = 0; a.mbBytes = 0;
+    a.count = 0; a.code = 0; a.mbBytes = 0; a.runs = nullptr;
     if (a.fz0 > a.fz1 || a.fx0 > a.fx1 || a.fy0 > a.fy1) {
         if (threadIdx.x == 0)
             __hip_atomic_store(flags + m.flag, (serial << 32) | 0xffffffffull,
@@ -125,7 +125,7 @@ __global__ void batch_mb_args_kernel(const BatchGrid* __restrict__ grids,
     a.stamp = count ? g.stamp : nullptr;
     a.lastchg = g.lastchg;
     a.count = count; a.code = stamp_code(count);
-    a.mbBytes = g.mbBytes;
+    a.mbBytes = g.mbBytes; a.runs = nullptr;
     args[i] = a;
 }
 
@@ -303,7 +303,7 @@ extern "C" int fteik_k_batch_mb_sweep(const BatchGrid* grids, int ngrids,
     // count: number of the iteration sweep in the record, 0 without one
     if (!chunk) count = 0;
     const void* fn = chunk
-        ? fteik_k_chunk_fn(fp32, count, cube)
+        ? fteik_k_chunk_fn(fp32, count, 1, cube)
         : linit
         ? (fp32 ? batch_mb_fn<float, true>(tile)
                 : batch_mb_fn<double, true>(tile))

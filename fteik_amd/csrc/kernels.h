@@ -43,6 +43,17 @@ struct SweepLaunch {
     // sweep chains: progress words of the two workgroup sets
     // (2*max_flags, zeroed once; serials only grow)
     unsigned long long* prog;
+    // chunk: iteration sweeps with the chunked tiles (sweep_chunk.h); their
+    // change record (fteik_k_stamp_bytes bytes; null: no chunk skipping),
+    // last changing sweep, number of this iteration sweep, and the tiles'
+    // run words (fteik_k_run_words, zeroed once; serials only grow)
+    int chunk;
+    unsigned long long* runs;
+    unsigned char* stamp;
+    unsigned* lastchg;
+    unsigned count;
+    unsigned mbBytes;            // bytes of mbx and, following it, mby
+    int cube;                    // equal spacings
 };
 
 // One grid of a batched solve (batch3d.hip); device pointers.
@@ -55,7 +66,7 @@ struct BatchGrid {
     unsigned long long* mby;       // per-node one), as SweepLaunch::mbx/mby
     int mbnt;
     int nz, nx, ny, zsi, xsi, ysi;
-    unsigned char* stamp;          // chunked tiles' change record
+    unsigned char* stamp;          // chunked tiles, as in SweepLaunch
     unsigned* lastchg;
     unsigned mbBytes;
 };
@@ -127,9 +138,10 @@ int fteik_k_batch_mb_sweep(const fteik::BatchGrid* grids, int ngrids,
 // sweep_chunk.hip: the chunked tiles' kernels (count: number of the sweep
 // in the record, 0 without one; cube: every grid has equal spacings),
 // whether a grid can use them (mbBytes: of its edge-major mailboxes), the
-// bytes of its change record
+// bytes of its change record and the words of its tiles' runs
 int fteik_k_chunk_fits(int nz, int nx, int ny, size_t mbBytes);
-const void* fteik_k_chunk_fn(int fp32, unsigned count, int cube);
+size_t fteik_k_run_words(int nx, int ny);
+const void* fteik_k_chunk_fn(int fp32, unsigned count, int batch, int cube);
 size_t fteik_k_stamp_bytes(long ngrd);
 long fteik_k_stamp_offset(void);
 // sweep3d.hip

@@ -12,7 +12,7 @@
 #include <hip/hip_runtime.h>
 #include <cstring>
 #include <stdint.h>
-#include "sweep_pencil.h"
+#include "sweep_chunk.h"
 
 namespace fteik {
 
@@ -355,6 +355,8 @@ static int launch_sweep_t(const SweepLaunch& L, int sweep, bool linit,
     a.mb = L.mb;
     a.mbx = L.mbx; a.mby = L.mby; a.mbnt = L.mbnt;
     a.colmod = nullptr; a.plan = nullptr;
+    a.stamp = nullptr; a.lastchg = nullptr;
+    a.count = 0; a.code = 0; a.mbBytes = 0; a.runs = nullptr;
     if (a.fz0 > a.fz1 || a.fx0 > a.fx1 || a.fy0 > a.fy1) return 0;
     if (L.schedule == 1) {
         const int nlev = (a.fz1 + a.fx1 + a.fy1) - (a.fz0 + a.fx0 + a.fy0) + 1;
@@ -370,6 +372,25 @@ static int launch_sweep_t(const SweepLaunch& L, int sweep, bool linit,
                                    dim3(256), 0, stream, a, Lv);
         }
         return hipGetLastError() == hipSuccess ? 0 : 1;
+    }
+    if (L.chunk && !linit) {
+        // the chunked tiles are for iteration sweeps (with the
+        // initialization sweeps' extra operator they would spill registers)
+        if (!L.mbx || !L.mby || !L.runs) return 2;
+        a.nbx = (a.fx1 - a.fx0 + CB)/CB;
+        a.nby = (a.fy1 - a.fy0 + CB)/CB;
+        const bool record = L.stamp && L.lastchg && L.count > 0;
+        a.stamp = record ? L.stamp + fteik_k_stamp_offset() : nullptr;
+        a.lastchg = L.lastchg;
+        a.count = L.count;
+        a.code = stamp_code(L.count);
+        a.mbBytes = L.mbBytes;
+        a.runs = L.runs;
+        void* args[] = {&a};
+        const hipError_t e = hipLaunchKernel(
+            fteik_k_chunk_fn(L.fp32, record ? L.count : 0, 0, L.cube),
+            dim3(a.nbx*a.nby), dim3(192), args, 0, stream);
+        return e == hipSuccess ? 0 : 1;
     }
     const int tile = (L.tile >= 0 && L.tile < kNumTiles) ? L.tile : 0;
     const TileShape ts = kTiles[tile];

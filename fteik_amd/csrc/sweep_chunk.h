@@ -38,6 +38,12 @@
 // 50 -> 31 ms; the batch in mixed precision 84 -> 40 ms.  What bounds a tile
 // is the issue rate of FP64 instructions in its active chunks and, where
 // little is left to do, a mailbox round trip per skipped chunk.
+// Three waves, single grids: a level of a lone tile 0.48 us (streamed tiles
+// 0.68), a dense 257^3 sweep 625 us (735), its solve of 19 iterations 104 ->
+// 84 ms, 101^3 with 2 iterations 6.3 -> 5.3 ms.  A dense sweep is its chain
+// of chunks (193 at 1.9 us) and a hop of 4 us, a chunk and the mailbox, for
+// each of 62 tiles from corner to corner; a sweep with nothing left to do is
+// the hops.
 #pragma once
 #include "sweep_pencil.h"
 
@@ -367,11 +373,15 @@ struct ChunkTile {
         e0.load(bmb, in_box(t0, hdepM) ? hent + t*hn*EB : kOut);
         e1.load(bmb, in_box(t0, cdepM) ? cent + t*a.ny*EB : kOut);
     }
-    __device__ bool ready(int t0, const MbEntry<R>& e0,
-                          const MbEntry<R>& e1) const
+    // clean: upwind tiles (bit 0 in x, 1 in y, 2 in both) whose entries for
+    // the chunk need not have been posted
+    __device__ bool ready(int t0, const MbEntry<R>& e0, const MbEntry<R>& e1,
+                          int clean) const
     {
-        return __ballot((in_box(t0, hdepM) && !e0.is(tag)) ||
-                        (in_box(t0, cdepM) && !e1.is(tag))) == 0;
+        return __ballot((in_box(t0, hdepM) && !e0.is(tag) &&
+                         !(clean & (hx ? 1 : 2))) ||
+                        (in_box(t0, cdepM) && !e1.is(tag) &&
+                         !(clean & 4))) == 0;
     }
     // field values (and change bytes) of the lanes without a mailbox; only
     // tiles on the box's first row of tiles along an axis have such lanes
@@ -454,6 +464,45 @@ struct ChunkTile {
              (in_box(t0, cdepD) && dirty_byte(b1));
     }
 
+    // Marks (in LDS, a byte per chunk) the chunks with a dirty node in the
+    // tile's columns or in the upwind columns without a mailbox: columns 0
+    // .. 63, then 64 .. 71 (before it in x), 72 .. 79 (in y) and 80.  A lane
+    // reads 16 bytes of a column at a time, consecutive lanes consecutive
+    // pieces.
+    __device__ void scan(unsigned char* dirt, int ng) const
+    {
+        // nodes fi = ez0 .. fz1, in memory order from byte lo of a column
+        const unsigned lo = (a.sz > 0) ? ez0 : a.nz - 1 - fz1;
+        const int n = (int) nbox + 1, np = (n + 15)/16;
+        const int total = (cdir ? 81 : 64)*np;
+        #pragma unroll 4
+        for (int p0 = 0; p0 < total; p0 += 64) {
+            const int p = p0 + lane, col = p/np, o = (p - col*np)*16;
+            const int cj = col < 64 ? fj0 + (col & 7)
+                         : col < 72 || col == 80 ? fj0 - 1 : fj0 + (col & 7);
+            const int ck = col < 64 ? fk0 + (col >> 3)
+                         : col < 72 ? fk0 + (col & 7) : fk0 - 1;
+            bool use = p < total && cj <= a.fx1 && ck <= a.fy1;
+            if (col >= 64)
+                use = use && (col < 72 ? fbx == 0 : col < 80 ? fby == 0 : cdir);
+            const unsigned base = column(min(max(cj, 0), a.fx1),
+                                         min(max(ck, 0), a.fy1))/SZ + lo;
+            unsigned w[4] = {0, 0, 0, 0};
+            if (use) __builtin_memcpy(w, a.stamp + base + o, 16);
+            unsigned m = 0;
+            #pragma unroll
+            for (int q = 0; q < 16; q++)
+                m |= dirty_byte((w[q >> 2] >> (8*(q & 3))) & 255) ? 1u << q
+                                                                  : 0u;
+            for (; m; m &= m - 1) {
+                const int q = o + __ffs((int) m) - 1;
+                if (q >= n) break;
+                const int fi = (a.sz > 0) ? ez0 + q : fz1 - q;
+                const int g = (fi + cj + ck - tlo) >> 2;      // or below 0
+                if (g >= -1 && g < ng) dirt[g + 1] = 1;
+            }
+        }
+    }
     // ---- results.  Posts the chunk's last column and last row (lanes
     // 0..31: row hc of the last column, 32..63: column hc of the last row;
     // step hq); rows: the chunk's ring rows, own: a column's dirty steps
@@ -626,7 +675,7 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
         // ---- the upwind neighbours' chunk
         {
             unsigned spins = 0;
-            while (!T.ready(t0, e0, e1)) {
+            while (!T.ready(t0, e0, e1, 0)) {
                 if (++spins > kSpinLimit) {
                     if (lane == 0) atomicExch(a.err, 1);
                     return;
@@ -724,6 +773,409 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
         prevDirty = SKIP && __ballot(nextDirty) != 0;
     }
     T.template finish<RECORD>(dmax, changed);
+}
+
+// -------------------------------------------------------- three waves
+// The same tile by three waves: the first computes and touches LDS only, the
+// second loads (mailbox, change record, old times, cells) and decides which
+// chunks are computed, the third posts and stores.  A wave's loads and
+// stores are counted together and complete in order, so a wave that polls
+// the mailbox after posting waits for its own stores to reach memory; here
+// the polling wave stores nothing.  For single grids, whose tiles leave
+// room for it; in a batch, where every SIMD has its waves of other tiles,
+// one wave per tile is faster.
+//
+// Buffers of three chunks in turn (chunk g in part g mod 3): ring rows, old
+// times, new cell layers, own dirty and changed steps.  Counters, one per
+// wave: g_load, g_comp, g_store = the chunks that wave is done with.  The
+// loading wave announces chunks one by one or, where nothing is dirty, a run
+// at once (s_news).
+//
+// Runs.  a.runs has a word per tile, each in a cache line of its own (the
+// tiles' polls and posts of words in shared lines got in each other's way:
+// 90.6 against 84.2 ms per 257^3 solve): (serial << 32) | first << 16 | end,
+// the tile's current run of chunks that it skips with no dirty node of its
+// own.
+// A tile whose own chunks are clean (s_dirt, from the change record, read
+// once) and whose upwind tiles' runs cover the same levels skips them all at
+// once, so a clean stretch costs one exchange per tile instead of one per
+// chunk.  When a run ends before the tile does, its entries are posted too,
+// for readers that come when a later run has replaced the word.
+constexpr int kRunStride = 16;          // words
+constexpr int kMaxDirt = 1024;          // chunks of s_dirt: nz up to 4000
+constexpr int kNews = 64;
+enum : int { kSkipClean = 0, kSkipDirty = 1, kCompute = 2 };
+template <typename R, bool SKIP, bool RECORD, bool CUBE>
+__device__ __forceinline__ void chunk3_body(const SweepArgs<R>& a,
+                                            const int wg)
+{
+    __shared__ R ring[12*CROW];
+    __shared__ R cbuf[12*CROW];
+    __shared__ R tbuf[3*CK*CTROW];
+    __shared__ unsigned char s_own[3][64], s_chg[3][64];
+    // announcement k in slot k mod kNews: what becomes of the next chunks,
+    // kSkipClean (nothing dirty of its own), kSkipDirty (see s_own) or
+    // kCompute, and, from bit 2 on, how many they are; the chunk it starts
+    // at; s_any, per part: whether the chunk changed a node on its steps 1..3
+    __shared__ int s_news[kNews], s_start[kNews], s_any[3];
+    __shared__ unsigned char s_dirt[SKIP ? kMaxDirt : 1];
+    __shared__ int g_load, g_comp, g_store, s_abort;
+    const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
+    const ChunkTile<R> T(a, wg, lane, RECORD);
+    if (T.empty() || (SKIP && sweep_is_clean(a))) return;     // uniform
+    if (threadIdx.x == 0) g_load = g_comp = g_store = s_abort = 0;
+    __syncthreads();
+    const int ng = (T.thi - T.tlo)/CK + 1;
+    auto give_up = [&]() {
+        if (lane == 0) {
+            atomicExch(a.err, 1);
+            __hip_atomic_store(&s_abort, 1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    };
+    // LDS accesses of a wave are in order, and a counter is written after
+    // the data it announces; a waiting wave reads it before them.  Returns
+    // the count, at least g, or -1 after a failure.
+    auto wait = [&](int* p, int g) -> int {
+        unsigned spins = 0;
+        int v;
+        while ((v = __builtin_amdgcn_readfirstlane(lds_load_rx(p))) < g) {
+            if (lds_load_rx(&s_abort)) return -1;
+            if (++spins > kSpinLimit) { give_up(); return -1; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        wave_lds_fence();
+        return v;
+    };
+    auto done = [&](int* p, int g) {
+        wave_lds_fence();
+        if (lane == 0)
+            __hip_atomic_store(p, g, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    };
+    // announcement k, of the chunks from g on
+    auto news = [&](int k, int g, int& f, int& n) {
+        if (!SKIP) { f = kCompute; n = 1; return; }
+        const int w = __builtin_amdgcn_readfirstlane(s_news[k & (kNews - 1)]);
+        f = w & 3;
+        n = w >> 2;
+    };
+    if (role == 0) {
+        // -------------------------------------------------------- compute
+        const Consts<R> c = chunk_consts<R, CUBE>(a);
+        ChunkPast<R> past = {R(0), R(0), R(0), R(0)};
+        bool loaded = false;
+        int part = 0, before = 2, avail = 0;
+        for (int g = 0, k = 0; g < ng; k++) {
+            if (avail <= g && (avail = wait(&g_load, g + 1)) < 0) return;
+            int f, n;
+            news(k, g, f, n);
+            if (f == kCompute) {
+                const int t0 = T.tlo + g*CK;
+                R* const rc = ring + part*4*CROW;
+                const R* const rp = ring + before*4*CROW;
+                if (!loaded) {
+                    past.w = rp[2*CROW + T.me - 1];
+                    past.s = rp[2*CROW + T.me - 9];
+                    past.sw = rp[CROW + T.me - 10];
+                    past.v = rp[3*CROW + T.me];
+                }
+                const unsigned chg = chunk_levels<R, CUBE, SKIP>(
+                    T, c, t0, rp, rc, cbuf + before*4*CROW,
+                    cbuf + part*4*CROW, tbuf + part*CK*CTROW, past, []() {});
+                if (SKIP) {
+                    s_chg[part][lane] = (unsigned char) chg;
+                    const bool any = __ballot(chg & 14u) != 0;
+                    if (lane == 0) s_any[part] = any ? 1 : 0;
+                }
+            }
+            loaded = f == kCompute;
+            g += n;
+            done(&g_comp, g);
+            part = g % 3;
+            before = part == 0 ? 2 : part - 1;
+        }
+    } else if (role == 1) {
+        // ----------------------------------------------------------- load
+        MbEntry<R> e0, e1;
+        R d0 = R(0), d1 = R(0);
+        int b0 = 0, b1 = 0;
+        unsigned stn = 0;
+        // runs of the upwind tiles (lanes 0, 1, 2: in x, y and both; none:
+        // a tile that always covers)
+        unsigned long long run = 0;
+        const int ux = T.fbx - (lane == 1 ? 0 : 1),
+                  uy = T.fby - (lane == 0 ? 0 : 1);
+        const bool up = SKIP && lane < 3 && ux >= 0 && uy >= 0;
+        const int uoff = lane == 2 ? 4 : 2;      // its chunk of our chunk 0
+        const unsigned long long* const upw = a.runs + kRunStride*(up ? ux*a.nby + uy
+                                                         : 0);
+        // tiles have runs: the chunks of a whole tile fit s_dirt
+        const bool runs = SKIP && ((int) T.nbox + 2*CB - 2)/CK < kMaxDirt - 1;
+        auto load_run = [&]() {
+            if (runs && up)
+                run = __hip_atomic_load(upw, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+        };
+        // end (in this tile's chunks) of the stretch from chunk g on that the
+        // upwind tiles' runs cover; g if none
+        // (clean: those that do)
+        int clean = 0;
+        auto covered = [&](int g) -> int {
+            if (!runs) return g;
+            const int b = (int) (run & 0xffffu) - uoff,
+                      f = (int) ((run >> 16) & 0xffffu) - uoff;
+            const bool mine = (unsigned) (run >> 32) == (unsigned) a.serial &&
+                              f <= g && b > g;
+            clean = (int) __ballot(up && mine);
+            // the box's other upwind columns have no tile: s_dirt
+            int end = up ? (mine ? b : g) : 1 << 20;
+            end = min(end, __shfl_xor(end, 1, 64));
+            end = min(end, __shfl_xor(end, 2, 64));
+            return min(__builtin_amdgcn_readfirstlane(end), ng);
+        };
+        // loaded: the chunk's old times and cells are on the way (tnx, cnx)
+        bool prevDirty = false, loaded = false;
+        int part = 2, before = 1, k = 0;
+        int first = -1;              // of the run that chunk g continues
+        R tnx[4], cnx[CNC];
+        if (SKIP) stn = T.load_stamp(T.tlo - CK);
+        T.load_entries(T.tlo - CK, e0, e1);
+        T.load_direct(T.tlo - CK, SKIP, d0, d1, b0, b1);
+        load_run();
+        if (runs) {
+            for (int i = lane; i <= ng; i += 64) s_dirt[i] = 0;
+            wave_lds_fence();
+            T.scan(s_dirt, ng);
+            wave_lds_fence();
+        }
+        auto announce = [&](int g, int f, int n) -> bool {
+            if (SKIP) {
+                // the slots of announcements long ago have been read
+                if ((k & 15) == 0 && k >= 48) {
+                    const int old = __builtin_amdgcn_readfirstlane(
+                        s_start[(k - 32) & (kNews - 1)]);
+                    if (wait(&g_comp, old) < 0 || wait(&g_store, old) < 0)
+                        return false;
+                }
+                if (lane == 0) {
+                    s_news[k & (kNews - 1)] = f | n << 2;
+                    s_start[k & (kNews - 1)] = g;
+                }
+            }
+            k++;
+            done(&g_load, g + n);
+            return true;
+        };
+        // the run's word: chunks from .. end - 1 continue or begin it
+        auto publish = [&](int from, int end) {
+            if (first < 0) first = from;
+            if (lane == 0)
+                __hip_atomic_store(a.runs + kRunStride*wg, (a.serial << 32) |
+                                   (unsigned long long) first << 16 |
+                                   (unsigned long long) end,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        for (int g = -1; g < ng; ) {
+            const int t0 = T.tlo + g*CK;
+            // ---- what does not need the neighbours: the own dirty nodes
+            // among those the chunk reads (steps t0 - 3 .. t0 + 2), and its
+            // old times and cells
+            unsigned own = 0;
+            bool active = g >= 0;
+            if (SKIP) {
+                own = T.own_dirty(t0, stn);
+                active = g >= 0 && (prevDirty || __ballot(own & 7u) != 0);
+            }
+            auto load_all = [&]() -> bool {
+                // of this chunk, and the three steps before it
+                R* const rp = ring + before*4*CROW;
+                R hist[3], pv0, pv1, x0 = R(0), x1 = R(0), cfirst[CNC];
+                int y0, y1;
+                MbEntry<R> p0, p1;
+                T.fetch_c(t0 - CK, cfirst);
+                T.fetch_hist(t0, hist);
+                T.fetch_t(t0, tnx);
+                T.fetch_c(t0, cnx);
+                T.load_entries(t0 - CK, p0, p1);
+                T.load_direct(t0 - CK, false, x0, x1, y0, y1);
+                T.halo_values(t0 - CK, p0, p1, x0, x1, pv0, pv1);
+                // no chunk before this one still needs its part
+                if (g > 0 && (wait(&g_store, g) < 0 || wait(&g_comp, g) < 0))
+                    return false;
+                T.park_c(cbuf + before*4*CROW, cfirst);
+                #pragma unroll
+                for (int q = 0; q < 3; q++)
+                    rp[(q + 1)*CROW + T.me] = hist[q];
+                rp[T.hq*CROW + T.hpos] = pv0;
+                if (lane < 4) rp[lane*CROW] = pv1;
+                T.park_t(tbuf + part*CK*CTROW, tnx);
+                T.park_c(cbuf + part*4*CROW, cnx);
+                return true;
+            };
+            bool parked = false;
+            if (g >= 0 && loaded) {
+                // this part's last chunk is stored, and the chunk before the
+                // last no longer reads its cell rows
+                if (wait(&g_store, g - 2) < 0 || wait(&g_comp, g - 1) < 0)
+                    return;
+                T.park_t(tbuf + part*CK*CTROW, tnx);
+                T.park_c(cbuf + part*4*CROW, cnx);
+                parked = true;
+            } else if (active) {
+                if (!load_all()) return;
+                parked = true;
+            }
+
+            // ---- the upwind neighbours' chunk
+            int end = covered(g);
+            {
+                unsigned spins = 0;
+                if (end <= g && !T.ready(t0, e0, e1, clean)) do {
+                    if (lds_load_rx(&s_abort)) return;
+                    if (++spins > kSpinLimit) { give_up(); return; }
+                    load_run();
+                    T.load_entries(t0, e0, e1);
+                    end = covered(g);
+                } while (end <= g && !T.ready(t0, e0, e1, clean));
+            }
+            // ---- a run: the covered chunks up to the first with a dirty
+            // node of its own
+            if (runs && !active && !loaded && end > g) {
+                int n = 0;
+                for (;; n += 64) {
+                    const int at = g + n + lane;
+                    const unsigned long long m = __ballot(
+                        at >= end || s_dirt[min(at, ng - 1) + 1]);
+                    if (m == 0) continue;
+                    n += __ffsll((long long) m) - 1;
+                    break;
+                }
+                if (n > 0) {
+                    const int from = max(g, 0);
+                    g += n;
+                    if (g > from) {
+                        publish(from, g);
+                        if (!announce(from, kSkipClean, g - from)) return;
+                    }
+                    part = g % 3;
+                    before = part == 0 ? 2 : part - 1;
+                    if (g < ng) {
+                        stn = T.load_stamp(T.tlo + g*CK);
+                        load_run();
+                        T.load_entries(T.tlo + g*CK, e0, e1);
+                        T.load_direct(T.tlo + g*CK, true, d0, d1, b0, b1);
+                    }
+                    continue;
+                }
+            }
+            // late: the halo's dirty nodes are looked at after the chunk has
+            // been announced
+            bool hd = true, cd = true, nextDirty = false, late = false;
+            if (SKIP) {
+                if (!active) T.halo_dirty(t0, e0, e1, b0, b1, hd, cd);
+                const bool known = active;
+                if (!active && g >= 0) {
+                    active = __ballot((hd && T.hq < 3) ||
+                                      (cd && lane < 3)) != 0;
+                    if (!active && loaded) {
+                        // dirty only if the chunk before changed a node
+                        if (wait(&g_comp, g) < 0) return;
+                        active = __builtin_amdgcn_readfirstlane(s_any[before])
+                                 != 0;
+                    }
+                }
+                if (active && !parked && !load_all()) return;
+                late = known;
+            }
+            if (active) {
+                R* const rc = ring + part*4*CROW;
+                R v0, v1;
+                T.halo_values(t0, e0, e1, d0, d1, v0, v1);
+                rc[T.hq*CROW + T.hpos] = v0;
+                if (lane < 4) rc[lane*CROW] = v1;
+            }
+            if (g >= 0) {
+                int f = kCompute;
+                if (SKIP) {
+                    const bool od = __ballot(own != 0) != 0;
+                    if (!active) f = od || !runs ? kSkipDirty : kSkipClean;
+                    if (f == kSkipDirty && wait(&g_store, g - 2) < 0) return;
+                    if (f != kSkipClean)
+                        s_own[part][lane] = (unsigned char) own;
+                }
+                if (f == kSkipClean) publish(g, g + 1);
+                else first = -1;
+                if (!announce(g, f, 1)) return;
+            }
+            if (SKIP) {
+                if (late) T.halo_dirty(t0, e0, e1, b0, b1, hd, cd);
+                nextDirty = (own & 14u) || (hd && T.hq > 0) ||
+                            (cd && lane > 0);
+            }
+            if (g + 1 < ng) {
+                if (SKIP) stn = T.load_stamp(t0 + CK);
+                load_run();
+                T.load_entries(t0 + CK, e0, e1);
+                T.load_direct(t0 + CK, SKIP, d0, d1, b0, b1);
+                if (active) {
+                    T.fetch_t(t0 + CK, tnx);
+                    T.fetch_c(t0 + CK, cnx);
+                }
+            }
+            loaded = active;
+            prevDirty = SKIP && __ballot(nextDirty) != 0;
+            g++;
+            before = part;
+            part = part == 2 ? 0 : part + 1;
+        }
+    } else {
+        // ---------------------------------------------------------- store
+        R dmax = R(0);
+        bool changed = false;
+        int part = 0, avail = 0;
+        int first = -1;           // of the clean chunks not yet posted
+        for (int g = 0, k = 0; g < ng; k++) {
+            if (avail <= g && (avail = wait(&g_load, g + 1)) < 0) return;
+            int f, n;
+            news(k, g, f, n);
+            const int t0 = T.tlo + g*CK;
+            if (f == kSkipClean) {
+                if (first < 0) first = g;
+                g += n;
+                done(&g_store, g);
+                part = g % 3;
+                continue;
+            }
+            if (SKIP && first >= 0) {
+                for (int i = first; i < g; i++)
+                    T.post(T.tlo + i*CK, false, nullptr, 0u);
+                first = -1;
+            }
+            const bool act = f == kCompute;
+            if (act && wait(&g_comp, g + 1) < 0) return;
+            const R* const rc = ring + part*4*CROW;
+            unsigned own = 0;
+            if (SKIP) {
+                own = s_own[part][T.post_lane()];
+                if (act) own |= s_chg[part][T.post_lane()];
+            }
+            T.post(t0, act, rc, own);
+            R out[4], old[4];
+            if (act) {
+                const R* const tb = tbuf + part*CK*CTROW;
+                #pragma unroll
+                for (int i = 0; i < 4; i++)
+                    old[i] = tb[T.lq*CTROW + 16*i + T.lc];
+                T.collect(rc, out);
+            }
+            done(&g_store, ++g);
+            if (act) T.template store<RECORD>(t0, old, out, dmax, changed);
+            part = part == 2 ? 0 : part + 1;
+        }
+        T.template finish<RECORD>(dmax, changed);
+    }
 }
 
 } // namespace fteik

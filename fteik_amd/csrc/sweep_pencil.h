@@ -170,6 +170,7 @@ struct SweepArgs {
     unsigned count;
     int code;
     unsigned mbBytes;            // of mbx and, after it, mby
+    unsigned long long* runs;    // run words of a single sweep's tiles
 };
 
 // The per-sweep values of a mailbox sweep, kept apart from SweepArgs so a

@@ -121,8 +121,14 @@ void fteik_solver3d_setMixedParameters(double bias, int maxCorrections,
  * workgroups can be resident; mailbox tiles (modes 1, 2) also launch
  * without co-residency: tiles are dealt to workgroups so that a tile waits
  * only on tiles of lower-numbered workgroups, and workgroups are dispatched
- * in order, so the lowest unfinished tile is always resident.  Every wait has a spin limit; a sweep that exceeds it
- * fails the solve with ierr = 1 rather than hanging. */
+ * in order, so the lowest unfinished tile is always resident.  Every wait
+ * has a spin limit; a sweep that exceeds it fails the solve with ierr = 1
+ * rather than hanging.  Until a shape is chosen the shapes that getTile
+ * reports serve the initialization sweeps, and the iterations run on chunked
+ * 8 x 8 tiles, which skip nodes that cannot change (grids too large for
+ * 32-bit offsets, or no memory for the change record: the reported shapes
+ * serve every sweep).  autotune keeps the chunked tiles if they are faster
+ * than every shape. */
 void fteik_solver3d_setTile(int tile, int tile32, int *ierr);
 void fteik_solver3d_getTile(int *tile, int *tile32, int *ntiles, int *ierr);
 /* EXTENSION: the autotuner.  Solves source isrc (1-based) once with every
@@ -135,7 +141,8 @@ void fteik_solver3d_autotune(int isrc, int *tile, int *tile32, int *ierr);
  * pipelined sweep whose columns have not changed since its last pass in the
  * same direction and whose upwind tiles are skipped too: such a pass would
  * reproduce the tile's values exactly, so results are unchanged (on by
- * default; mailbox tile shapes only). */
+ * default; mailbox tile shapes only).  The chunked tiles skip by node:
+ * chunks of four levels without a changed upwind neighbour. */
 void fteik_solver3d_setTileSkipping(int on, int *ierr);
 /* EXTENSION: run the Gauss-Seidel iteration sweeps of a solve as one chain
  * in which each sweep starts while the one before it is still running,

@@ -1,5 +1,5 @@
-"""The chunked tiles of a batch's iteration sweeps (the default until a tile
-shape is chosen): fields equal the oracle's bit for bit, and the streamed tiles'
+"""The chunked tiles of the iteration sweeps (the default until a tile shape
+is chosen): fields equal the oracle's bit for bit, and the streamed tiles'
 where the oracle has no such mode, at the edges of tiles (8 x 8 columns),
 chunks (4 levels) and runs (4,092 levels), with and without skipping."""
 from ctypes import byref, c_int
@@ -36,6 +36,50 @@ def _oracle(vel, nz, nx, ny, d, src, nsweep):
     slow = orc.cell_slowness(vel, nz, nx, ny, order=0)
     s = orc.source_locate((nz, nx, ny) + d + (0.0, 0.0, 0.0), *src, slow)
     return orc.solve3d(slow, nz, nx, ny, *d, s, nsweep, 3.0, schedule=1)
+
+
+def _solver(case, seed, precision=0, skipping=1, tile=None, conv=0.0):
+    nz, nx, ny, d, c, nsweep = case
+    L, ierr = lib(), c_int(1)
+    L.fteik_solver3d_initialize(nz, nx, ny, 0.0, 0.0, 0.0, *d, nsweep, 3.0,
+                                conv, 0, byref(ierr))
+    assert ierr.value == 0
+    L.fteik_solver3d_setPrecision(precision, byref(ierr))
+    L.fteik_solver3d_setTileSkipping(skipping, byref(ierr))
+    if tile is not None:
+        L.fteik_solver3d_setTile(tile, tile, byref(ierr))
+        assert ierr.value == 0
+    vel = _model(nz, nx, ny, seed)
+    src = tuple(a * b for a, b in zip(c, d))
+    L.fteik_solver3d_setVelocityModel64f(vel.size, _d(vel), byref(ierr))
+    assert ierr.value == 0
+    s = [np.array([a]) for a in src]
+    L.fteik_solver3d_setSources64f(1, *[_d(a) for a in s], byref(ierr))
+    assert ierr.value == 0
+    L.fteik_solver3d_solveSourceLSM(1, byref(ierr))
+    assert ierr.value == 0
+    tt = np.zeros(nz * nx * ny)
+    L.fteik_solver3d_getTravelTimeField64f(tt.size, 0, _d(tt), byref(ierr))
+    assert ierr.value == 0
+    return tt, vel, src
+
+
+@pytest.mark.parametrize("skipping", [1, 0])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_chunked_sweeps_match_oracle(case, skipping):
+    c = CASES[case]
+    print("case: chunked", c, "skipping", skipping, flush=True)
+    tt, vel, src = _solver(c, 100 + case, skipping=skipping)
+    np.testing.assert_array_equal(tt, _oracle(vel, *c[:4], src, c[5]))
+
+
+@pytest.mark.parametrize("case", [1, 2, 4, 5])
+def test_chunked_mixed_matches_streamed(case):
+    c = CASES[case]
+    print("case: chunked mixed", c, flush=True)
+    a, _, _ = _solver(c, 200 + case, precision=1)
+    b, _, _ = _solver(c, 200 + case, precision=1, tile=12)
+    np.testing.assert_array_equal(a, b)
 
 
 @pytest.mark.parametrize("cube", [True, False])
