@@ -205,9 +205,7 @@ int fteik_k_solve2d(double* tt, const double* slow, int nz, int nx,
                     int zsi, int xsi, int nsweep, int nsrc_batch,
                     int ld_tt, const double* zsa_v, const double* xsa_v,
                     const int* zsi_v, const int* xsi_v, int schedule,
-                    int* err, double* scratch, hipStream_t stream);
-// doubles of scratch per source the pipelined 2D sweeps need
-constexpr int kSolve2dScratch = 512;
+                    int* err, hipStream_t stream);
 
 // locate.hip
 int fteik_k_tables_d2f(float* tables, const double* tt, int ngrd,
