@@ -23,7 +23,8 @@
 // 48 stations, 161 x 161 x 81 cells, 10,000 events: of 35,301 blocks and
 // 726 groups an event's search evaluates the 726 representatives, about 51
 // groups' blocks and 92 blocks' cells, 9,900 evaluations instead of
-// 2,099,601.  The call: 163 -> 4.3 ms (k_cells 1.31 ms and k_children 0.64
+// 2,099,601.  The call (from 8,193 events on it keeps the full search, see
+// kIndexEvents): 163 -> 4.3 ms (k_cells 1.31 ms and k_children 0.64
 // ms per 5,400 events, k_group 0.09); 1500 events on 37 tables of 41 x 90 x
 // 77, for which the full search makes a pass per event: 46.8 -> 0.68 ms;
 // one event on the 48 tables: 336 -> 105 us.  What bounds it is latency: a
