@@ -414,8 +414,8 @@ void fteik_solver3d_initialize(int nz, int nx, int ny, double z0, double x0,
     g3.cooperative = first >= 0;
     g3.tile = g3.tile32 = first >= 0 ? first : 0;
     // The iteration sweeps run on chunked tiles, which skip by node and not
-    // by tile: a solve of 24 x 32 x 28 nodes 2.2 -> 1.6 ms, 101^3 6.3 -> 5.3
-    // ms, 257^3 104 -> 84 ms, 129 x 257 x 257 in mixed precision 60 -> 49 ms
+    // by tile: a solve of 33 x 29 x 31 nodes 2.2 -> 1.6 ms, 101^3 6.3 -> 5.3
+    // ms, 257^3 104 -> 84 ms, 131 x 190 x 157 in mixed precision 60 -> 49 ms
     // (streamed tiles with tile skipping before).  The initialization sweeps
     // keep the tile above.
     g3.chunked = g3.chunkFits;

@@ -37,9 +37,9 @@ struct Batch3D {
     // tile on 64 grids of 64..192 per axis)
     int mbTile = 12, mapMbTile = -1;
     // until a tile shape is chosen, the iteration sweeps run on chunked
-    // tiles where every grid can use them (chunked): 64 grids of 20 .. 160
-    // per axis, converged, 98 -> 29 ms; 8 station tables of 129 x 129 x 65,
-    // 50 -> 31 ms
+    // tiles where every grid can use them (chunked): 16 grids of 64 .. 192
+    // per axis, 12 iterations, 98 -> 29 ms; 48 station tables of 81 x 161 x
+    // 161, 2 iterations, 50 -> 31 ms
     bool chunk = true, chunked = false, mapChunk = false;
     int mbOff[9] = {0}, mbN[9] = {0};
     unsigned long long *d_mb = nullptr;

@@ -33,9 +33,10 @@
 // skipped chunk posts entries without a value: a reader that needs one
 // takes it from the field, which this launch does not change there.  The
 // first eight sweeps of a record (RECORD without SKIP) compute every chunk.
-// Measured (one wave, batches): 64 grids of 20 .. 160 nodes per axis,
-// converged, 98 -> 29 ms (streamed tiles before); 8 tables of 129 x 129 x 65
-// 50 -> 31 ms; the batch in mixed precision 84 -> 40 ms.  What bounds a tile
+// Measured (one wave, batches): 16 grids of 64 .. 192 nodes per axis, 12
+// iterations, 98 -> 29 ms (streamed tiles before); 48 tables of 81 x 161 x
+// 161, 2 iterations, 50 -> 31 ms; 8 of the 16 grids in mixed precision 84 ->
+// 40 ms.  What bounds a tile
 // is the issue rate of FP64 instructions in its active chunks and, where
 // little is left to do, a mailbox round trip per skipped chunk.
 // Three waves, single grids: a level of a lone tile 0.48 us (streamed tiles
