@@ -725,8 +725,8 @@ void locate_setTravelTimeFieldFromBatch3d(int igrid, int itf, int *ierr)
         *ierr = 1;
         return;
     }
-    locator_tables_changed();
-    if (fteik_k_tables_d2f(gl.d_tab + (long) (itf - 1)*gl.ldgrd, x.d_tt,
+    if (!locator_tables_changed() ||
+        fteik_k_tables_d2f(gl.d_tab + (long) (itf - 1)*gl.ldgrd, x.d_tt,
                            gl.ngrd, g_dev.stream) != 0 || !sync_ok())
         *ierr = 1;
 }

@@ -122,8 +122,10 @@ struct Locator {
     std::vector<unsigned char> t0Skip;
 };
 extern Locator gl;
-// The locator's tables changed (their index is out of date).
-void locator_tables_changed();
+// Called before the locator's tables change: their index goes out of date,
+// and the origin-time work array takes what it still has to take from them.
+// false: GPU error.
+bool locator_tables_changed();
 
 int padlength32(int alignment, int n);
 float weight_norm(const float *w, int lntf);

@@ -45,6 +45,27 @@ float weight_norm(const float *w, int lntf)
     return 1.0f/s;
 }
 
+// Gives the origin-time work array the estimate of the last event located
+// through the index, which leaves the array as it was.  Runs before the
+// array is read and before the tables or their sizes change.
+bool settle_origin_times()
+{
+    if (!gl.t0Stale) return true;
+    gl.t0Stale = false;
+    const unsigned long long init = ~0ull;
+    if (h2d(gl.d_obs, gl.t0Obs.data(), gl.lntf*sizeof(float)) &&
+        h2d(gl.d_wt, gl.t0Wt.data(), gl.lntf*sizeof(float)) &&
+        h2d(gl.d_skip, gl.t0Skip.data(), (size_t) gl.lntf) &&
+        h2d(gl.d_best, &init, sizeof(init)) &&
+        fteik_k_locate(gl.d_tab, gl.ntf, gl.ngrd, gl.ldgrd, gl.d_obs,
+                       gl.d_wt, gl.d_skip, gl.lntf,
+                       weight_norm(gl.t0Wt.data(), gl.lntf), gl.d_t0,
+                       nullptr, 0, gl.d_best, g_dev.stream) == 0 &&
+        sync_ok()) return true;
+    msg("locate: GPU error while updating the origin times");
+    return false;
+}
+
 } // namespace fteik_capi
 
 extern "C" {
@@ -66,7 +87,8 @@ void locate_setNumberOfEvents(int nEvents, int *ierr)
 
 void locate_setNumberOfTravelTimeFields(int ntf, int *ierr)
 {
-    *ierr = 0;
+    *ierr = settle_origin_times() ? 0 : 1;
+    if (*ierr) return;
     gl.ntf = 0;
     if (ntf < 1) {
         printf("locate_setNumberOfTravelTimeFields: ntf=%4d must be positive\n",
@@ -79,7 +101,8 @@ void locate_setNumberOfTravelTimeFields(int ntf, int *ierr)
 
 void locate_setNumberOfGridPointsF(int ngrd, int *ierr)
 {
-    *ierr = 0;
+    *ierr = settle_origin_times() ? 0 : 1;
+    if (*ierr) return;
     gl.ngrd = 0;
     if (ngrd < 1) {
         printf("locate_setNumberOfGridPointsF: Number of grid points=%8d must "
@@ -158,8 +181,8 @@ void locate_setTravelTimeField64f(int ngrdIn, int itf, const double *tt,
         return;
     }
     if (!gl.d_tmp && !dalloc(&gl.d_tmp, gl.ngrd)) { *ierr = 1; return; }
-    locator_tables_changed();
-    if (!h2d(gl.d_tmp, tt, (size_t) gl.ngrd*sizeof(double)) ||
+    if (!locator_tables_changed() ||
+        !h2d(gl.d_tmp, tt, (size_t) gl.ngrd*sizeof(double)) ||
         fteik_k_tables_d2f(gl.d_tab + (long) (itf - 1)*gl.ldgrd, gl.d_tmp,
                            gl.ngrd, g_dev.stream) || !sync_ok()) *ierr = 1;
 }
@@ -185,8 +208,8 @@ void locate_setTravelTimeField32f(int ngrdIn, int itf, const float *tt,
         *ierr = 1;
         return;
     }
-    locator_tables_changed();
-    if (!h2d(gl.d_tab + (long) (itf - 1)*gl.ldgrd, tt,
+    if (!locator_tables_changed() ||
+        !h2d(gl.d_tab + (long) (itf - 1)*gl.ldgrd, tt,
              (size_t) gl.ngrd*sizeof(float))) *ierr = 1;
 }
 
@@ -307,19 +330,8 @@ void locate_locateEvent(int evnmbr, int *optIndx, double *t0Opt,
     }
     const float xnorm = weight_norm(gl.wt.data() + k, gl.lntf);
     const unsigned long long init = ~0ull;
-    if (gl.t0Stale && gl.refCompat) {
-        if (!h2d(gl.d_obs, gl.t0Obs.data(), gl.lntf*sizeof(float)) ||
-            !h2d(gl.d_wt, gl.t0Wt.data(), gl.lntf*sizeof(float)) ||
-            !h2d(gl.d_skip, gl.t0Skip.data(), (size_t) gl.lntf) ||
-            !h2d(gl.d_best, &init, sizeof(init)) ||
-            fteik_k_locate(gl.d_tab, gl.ntf, gl.ngrd, gl.ldgrd, gl.d_obs,
-                           gl.d_wt, gl.d_skip, gl.lntf,
-                           weight_norm(gl.t0Wt.data(), gl.lntf), gl.d_t0,
-                           nullptr, 0, gl.d_best, g_dev.stream) != 0) {
-            msg("locate_locateEvent: GPU error");
-            return;
-        }
-    }
+    // (without the reference's behaviour this event's estimate replaces it)
+    if (gl.refCompat && !settle_origin_times()) return;
     gl.t0Stale = false;
     bool ok = h2d(gl.d_obs, gl.obs.data() + k, gl.lntf*sizeof(float)) &&
               h2d(gl.d_wt, gl.wt.data() + k, gl.lntf*sizeof(float)) &&

@@ -258,10 +258,11 @@ bool worth_it(int n)
 
 namespace fteik_capi {
 
-void locator_tables_changed()
+bool locator_tables_changed()
 {
     gi.ready = gi.off = false;
     gi.searches = 0;
+    return settle_origin_times();
 }
 
 void index_release()
@@ -280,7 +281,7 @@ int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
         return 1;
     // sizes set after initialize are not those of the tables
     if (gi.ready && (gi.g.ntf != gl.ntf || gi.ngrd != gl.ngrd))
-        locator_tables_changed();
+        if (!locator_tables_changed()) return 2;
     for (int e = 0; e < n; e++)
         if ((size_t) evnmbr[e] > gl.plain.size() ||
             !gl.plain[(size_t) (evnmbr[e] - 1)]) return 1;

@@ -14,6 +14,8 @@ constexpr float kPlainLimit = 1.0e15f;
 // memory): search in full; 2: GPU error.
 int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
                  double *objOpt);
+// Brings the origin-time work array up to date (capi_locate.cpp).
+bool settle_origin_times();
 // Frees the index and its work space.
 void index_release();
 

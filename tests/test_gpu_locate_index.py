@@ -116,3 +116,48 @@ def test_index_left_out_for_infinite_times():
     tables = _tables(rng, 10, 30, 31, 32)
     tables[4, 12345] = np.inf
     _check(tables, _events(rng, tables, 60), searches=0)
+
+
+@pytest.mark.parametrize("change", ["table32", "table64", "sizes"])
+def test_origin_times_carry_over_from_the_old_tables(change):
+    """With the reference's compatibility an event starts from the origin
+    times that the event before it left, also where a table (or the number of
+    tables) changed in between and the earlier event went through the
+    index."""
+    print("case:", change, flush=True)
+    rng = np.random.default_rng(21)
+    ntf, shape = 32, (120, 120, 130)      # large: one event uses the index
+    tables = _tables(rng, ntf, *shape)
+    ngrd = tables.shape[1]
+    obs = _events(rng, tables, 2)
+    k, t, w = obs[0]
+    obs[0] = (k[:-1], t[:-1], w[:-1])     # no pick at the last table
+    L = lib()
+    f = L.fteik_k_locate_index_searches
+    f.restype = ctypes.c_int
+    loc = fa.Locator(2, ntf, ngrd)
+    ref = orc.Locator(2, ntf, ngrd)
+    for i in range(ntf):
+        loc.setTravelTimeField(i + 1, tables[i])
+        ref.set_table(i + 1, tables[i].astype(np.float64))
+    for e, (k, t, w) in enumerate(obs):
+        loc.setObservation(e + 1, k, t, w)
+        ref.set_observation(e + 1, k.astype(np.int32), t, w)
+    loc.setReferenceCompatibility(0)
+    for _ in range(2):                    # the second builds the index
+        got = loc.locateEvent(2)
+    assert f() == 1
+    assert got == ref.locate(2, accumulate_t0=True, pad_argmin=False)
+    if change == "sizes":
+        ierr = ctypes.c_int(1)
+        L.locate_setNumberOfTravelTimeFields(ntf - 1, ctypes.byref(ierr))
+        assert ierr.value == 0
+    else:
+        new = tables[0] * np.float32(1.3)
+        loc.setTravelTimeField(1, new if change == "table32"
+                               else new.astype(np.float64))
+        ref.set_table(1, new.astype(np.float64))
+    loc.setReferenceCompatibility(1)
+    assert loc.locateEvent(1) == ref.locate(1, accumulate_t0=True,
+                                            pad_argmin=True)
+    loc.finalize()
