@@ -40,6 +40,10 @@ using fteik::LocIndex;
 constexpr int EV = fteik::kLocEv;     // events a thread carries (k_group)
 constexpr float kEps = 1.1920929e-7f; // 2^-23
 constexpr float kRel = 1.0e-5f;       // relative slack of the bounds
+// Absolute slack: each of an objective's or a bound's at most 96 squares
+// loses up to 2^-126 where it underflows, which moves its root by up to
+// 1.5e-18, and kappa (below 10) multiplies the bound's.
+constexpr float kTiny = 1.0e-16f;
 
 __device__ __forceinline__ unsigned long long key_of(float obj, int cell)
 {
@@ -97,10 +101,13 @@ __device__ __forceinline__ float keep_norm(unsigned long long key)
 
 // Lower bound of |u| over a block: obj at its representative, s2 =
 // sum w^2 h^2; per event kap = kappa and mar, twice what rounding can move
-// a computed |u|.
+// a computed |u|.  An objective that overflowed says that it is at least the
+// largest number, not that its block holds no finite one.
 __device__ __forceinline__ float low_norm(float obj, float s2, float kap,
                                           float mar)
 {
+    const float big = 0.5f*FLT_MAX;
+    obj = obj > big ? big : obj;         // (a NaN stays one)
     return sqrtf(2.0f*obj)*(1.0f - kRel) - kap*sqrtf(s2)*(1.0f + kRel) - mar;
 }
 
@@ -286,7 +293,7 @@ void k_events(int n, int lntf, int ntf, int nt,
     // a computed residual is off by at most about (npick + 12) roundings of
     // the largest residual; twice that for each of the two cells compared
     const float rmax = omax + __uint_as_float(*tmax);
-    v.mar[e] = 4.0f*(float) (np + 16)*kEps*rmax*sqrtf(sw2);
+    v.mar[e] = 4.0f*(float) (np + 16)*kEps*rmax*sqrtf(sw2) + kTiny;
 }
 
 // --------------------------------------------------------------- search

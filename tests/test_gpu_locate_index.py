@@ -68,7 +68,7 @@ def _check(tables, obs, searches=1):
     loc.finalize()
 
 
-def _events(rng, tables, n, missing=0.0):
+def _events(rng, tables, n, missing=0.0, noise=0.1):
     ntf, ngrd = tables.shape
     out = []
     for c in rng.integers(0, ngrd, n):
@@ -77,7 +77,7 @@ def _events(rng, tables, n, missing=0.0):
         k = np.flatnonzero(have)
         w = rng.choice((1.0, 0.5, 0.1), k.size) if missing else np.ones(k.size)
         t = tables[k, c].astype(np.float64) + rng.uniform(0, 50) \
-            + rng.normal(0, 0.1, k.size)
+            + rng.normal(0, noise, k.size)
         out.append(((k + 1).astype(np.int32), t, w))
     return out
 
@@ -109,6 +109,21 @@ def test_index_on_other_tables(kind):
         tables = _tables(rng, ntf, 130, 151, 1)
     tables = np.ascontiguousarray(tables)
     _check(tables, _events(rng, tables, 60, 0.2))
+
+
+@pytest.mark.parametrize("scale,weight,noise,missing", [
+    (1000 * 10 ** (6 / 7), 0.99e15, 1.0, 0.0), (1.0e5, 0.99e15, 0.1, 0.2),
+    (1.0e6, 0.99e15, 0.1, 0.2), (10 ** (-25 / 3), 1.1e-14, 0.1, 0.2),
+    (1.0e-8, 1.01e-15, 1.0, 0.0), (10 ** -7.5, 1.01e-15, 1.0, 0.0),
+    (1.0e-6, 1.1e-14, 0.1, 0.2)])
+def test_index_at_the_ends_of_single_precision(scale, weight, noise, missing):
+    """Misfits that overflow at a block's representative but not in all of
+    its cells, and misfits of a few units of the smallest denormal."""
+    rng = np.random.default_rng(17)
+    tables = (_tables(rng, 9, 41, 37, 33) * np.float32(scale))
+    obs = [(k, t, w * weight) for k, t, w in
+           _events(rng, tables, 70, missing, noise=noise * scale)]
+    _check(tables, obs)
 
 
 def test_index_left_out_for_infinite_times():
