@@ -313,8 +313,10 @@ void locate_locateEvent(int evnmbr, int *optIndx, double *t0Opt,
     }
     const size_t k = (size_t) (evnmbr - 1)*gl.lntf;
     if (!gl.refCompat) {
-        const int rc = index_search(1, &evnmbr, optIndx, t0Opt, objOpt);
-        if (rc == 0) {
+        std::vector<int> redo;
+        const int rc = index_search(1, &evnmbr, optIndx, t0Opt, objOpt,
+                                    &redo);
+        if (rc == 0 && redo.empty()) {
             // the work array takes this event's estimate when it is next
             // read
             gl.t0Stale = true;
@@ -369,26 +371,10 @@ void locate_locateEvent(int evnmbr, int *optIndx, double *t0Opt,
     *objOpt = (double) obj;
 }
 
-void locate_locateEvents(int n, const int *evnmbr, int *optIndx,
-                         double *t0Opt, double *objOpt, int *ierr)
+// Every cell for events evnmbr[0..n-1]; false: GPU error.
+static bool full_search(int n, const int *evnmbr, int *optIndx,
+                        double *t0Opt, double *objOpt)
 {
-    *ierr = 0;
-    if (!gl.init || n < 1) {
-        msg("locate_locateEvents: locator not initialized or no events");
-        *ierr = 1;
-        return;
-    }
-    for (int e = 0; e < n; e++)
-        if (evnmbr[e] < 1 || evnmbr[e] > gl.nEvents) {
-            msg("locate_locateEvents: invalid event %d", evnmbr[e]);
-            *ierr = 1;
-            return;
-        }
-    {
-        const int rc = index_search(n, evnmbr, optIndx, t0Opt, objOpt);
-        if (rc == 2) { msg("locate_locateEvents: GPU error"); *ierr = 1; }
-        if (rc != 1) return;
-    }
     std::vector<float> o((size_t) n*gl.lntf), w((size_t) n*gl.lntf), xn((size_t) n);
     std::vector<unsigned char> sk((size_t) n*gl.lntf);
     for (int e = 0; e < n; e++) {
@@ -455,10 +441,47 @@ void locate_locateEvents(int n, const int *evnmbr, int *optIndx,
          d2h(t0v.data(), d_t0v, (size_t) n*sizeof(float));
     dfree(d_o); dfree(d_w); dfree(d_w2); dfree(d_xn); dfree(d_sk); dfree(d_c);
     dfree(d_t0v);
-    if (!ok) { msg("locate_locateEvents: GPU error"); *ierr = 1; return; }
+    if (!ok) return false;
     for (int e = 0; e < n; e++)
         t0Opt[e] = (double) t0v[(size_t) e]
                  + gl.tepoch[(size_t) (evnmbr[e] - 1)];
+    return true;
+}
+
+void locate_locateEvents(int n, const int *evnmbr, int *optIndx,
+                         double *t0Opt, double *objOpt, int *ierr)
+{
+    *ierr = 0;
+    if (!gl.init || n < 1) {
+        msg("locate_locateEvents: locator not initialized or no events");
+        *ierr = 1;
+        return;
+    }
+    for (int e = 0; e < n; e++)
+        if (evnmbr[e] < 1 || evnmbr[e] > gl.nEvents) {
+            msg("locate_locateEvents: invalid event %d", evnmbr[e]);
+            *ierr = 1;
+            return;
+        }
+    std::vector<int> redo;
+    const int rc = index_search(n, evnmbr, optIndx, t0Opt, objOpt, &redo);
+    bool ok = rc != 2;
+    if (rc == 1) {
+        ok = full_search(n, evnmbr, optIndx, t0Opt, objOpt);
+    } else if (ok && !redo.empty()) {
+        const size_t m = redo.size();
+        std::vector<int> ev(m), opt(m);
+        std::vector<double> t0(m), obj(m);
+        for (size_t q = 0; q < m; q++) ev[q] = evnmbr[redo[q]];
+        ok = full_search((int) m, ev.data(), opt.data(), t0.data(),
+                         obj.data());
+        for (size_t q = 0; q < m && ok; q++) {
+            optIndx[redo[q]] = opt[q];
+            t0Opt[redo[q]] = t0[q];
+            objOpt[redo[q]] = obj[q];
+        }
+    }
+    if (!ok) { msg("locate_locateEvents: GPU error"); *ierr = 1; }
 }
 
 void locate_computeStatics32fF(const int *ldo, const int *nobs,

@@ -15,6 +15,8 @@ struct Index {
     int ngrd = 0;                    // cells of the index
     int through = 0;                 // searches through the index
     int searches = 0;                // full searches since a table changed
+    int pause = 0;                   // searches of several events to come
+                                     // that are made in full
     fteik::LocIndex g;
     size_t permCap = 0, repCap = 0, srepCap = 0;   // floats
     // work space: events (floats each holds), pairs of a batch
@@ -33,6 +35,7 @@ void free_events()
     dfree(gi.v.o8); dfree(gi.v.w8); dfree(gi.v.h8); dfree(gi.v.row);
     dfree(gi.v.xn); dfree(gi.v.kap); dfree(gi.v.mar); dfree(gi.v.best);
     gi.v.t0 = nullptr;
+    gi.v.over = nullptr;
     dfree(gi.d_obs); dfree(gi.d_wt); dfree(gi.d_skip);
     gi.evCap = gi.evTf = gi.rawCap = 0;
 }
@@ -156,7 +159,7 @@ bool build()
     g.h = g.rep + nr/2;
     g.sh = g.srep + nsr/2;
     if ((!g.tmax && !dalloc(&g.tmax, 1)) ||
-        (!g.npair && !dalloc(&g.npair, 2))) return true;
+        (!g.npair && !dalloc(&g.npair, fteik::kLocCounts))) return true;
     unsigned tm = 0;
     if (hipMemsetAsync(g.tmax, 0, sizeof(unsigned), g_dev.stream)
             != hipSuccess ||
@@ -180,14 +183,14 @@ bool work_space(int n)
     if (ne > gi.evCap || tf > gi.evTf) {
         const long c = std::max(ne, gi.evCap), f = std::max(tf, gi.evTf);
         free_events();
-        // best and t0 adjoin: one copy brings both back
+        // best, t0 and over adjoin: one copy brings them back
         if (!dalloc(&gi.v.o8, (size_t) (c*f)) ||
             !dalloc(&gi.v.w8, (size_t) (c*f)) ||
             !dalloc(&gi.v.h8, (size_t) (c*f)) ||
             !dalloc(&gi.v.row, (size_t) (3*c*f)) ||
             !dalloc(&gi.v.xn, (size_t) c) || !dalloc(&gi.v.kap, (size_t) c) ||
             !dalloc(&gi.v.mar, (size_t) c) ||
-            !dalloc(&gi.v.best, (size_t) (c + (c + 1)/2)) ||
+            !dalloc(&gi.v.best, (size_t) (2*c)) ||
             !dalloc(&gi.d_obs, (size_t) (c*f)) ||
             !dalloc(&gi.d_wt, (size_t) (c*f)) ||
             !dalloc(&gi.d_skip, (size_t) (c*f))) {
@@ -199,6 +202,7 @@ bool work_space(int n)
         gi.evTf = f;
     }
     gi.v.t0 = (float *) (gi.v.best + n);
+    gi.v.over = (unsigned *) (gi.v.t0 + n);
     // pairs (group, event) of a batch of eb events
     const long per = (long) g.ns*(64 + 2 + 1)*(long) sizeof(float);
     long eb = std::max<long>(fteik::kLocEv, (long) kPairBytes/per
@@ -236,22 +240,49 @@ bool batch_kernel(int ntf)
            ntf == 56 || ntf == 64;
 }
 
+// Estimated time of the full search for n events (seconds).  The batched
+// kernel makes 51e12 operations a second, 9 per cell, table and event;
+// without it an event is a pass over the tables at 1.8 TB/s (measured 242 us
+// for 403 MB) and a launch.
+double full_time(int n)
+{
+    const double cells = (double) gl.ngrd*gl.ntf;
+    return (n > 1 && batch_kernel(gl.ntf))
+        ? 20e-6 + (double) n*cells*1.8e-13
+        : (double) n*(6e-6 + cells*4.0/1.8e12);
+}
+
 // Whether the estimated time of a search through the index is below that of
-// the full one (seconds).  Full: the batched kernel makes 51e12 operations a
-// second, 9 per cell, table and event; without it an event is a pass over
-// the tables at 1.8 TB/s (measured 242 us for 403 MB) and a launch.  Index:
-// about 90 us of launches and latencies, 0.3 us an event (measured 0.43 us
-// with 10,000 events, 105 us for one), and once per set of tables its
-// building, at first two passes over them (measured 340 us for 403 MB).
+// the full one: about 90 us of launches and latencies, 0.3 us an event
+// (measured 0.43 us with 10,000 events, 105 us for one), and once per set of
+// tables its building, at first two passes over them (measured 340 us for
+// 403 MB).  Picks that fit badly leave more blocks; see block_limit.
 bool worth_it(int n)
 {
     const double cells = (double) gl.ngrd*gl.ntf;
-    const double full = (n > 1 && batch_kernel(gl.ntf))
-        ? 20e-6 + (double) n*cells*1.8e-13
-        : (double) n*(6e-6 + cells*4.0/1.8e12);
     double index = 90e-6 + n*0.3e-6;
     if (!gi.ready && gi.searches == 0) index += 150e-6 + cells*8.0/1.5e12;
-    return index < full;
+    return index < full_time(n);
+}
+
+// Blocks whose evaluation takes as long as the full search of n events, or
+// ~0 where there are not as many: a batch of events with more blocks left
+// after the bounds is given up and searched in full.  A block's times pass
+// at 4.2 to 14 TB/s, the more the more events share it.  The full search
+// has, beyond full_time, allocations and copies of 0.3 ms a call and, with
+// more events than its few-event kernel takes, 0.5 ns a cell, and 0.3 ps a
+// cell and event whatever the number of tables.  4,096 events on 48 tables
+// of 81 x 161 x 161 (35,301 blocks, limit 13,800 an event): picks with an
+// outlier leave 630 blocks, picks without any relation to smooth tables
+// 3,950 (46 ms, in full 67); with 0.25 s of noise in every table value they
+// leave 17,100 (131 ms through the index).
+unsigned block_limit(int n)
+{
+    const double block = (double) gl.ntf*256.0/9e12;
+    const double more = 0.3e-3 + gl.ngrd*(n > 8 ? 0.5e-9 : 0.0)
+                      + (double) n*gl.ngrd*0.3e-12;
+    const double limit = (full_time(n) + more)/block;
+    return limit < (double) n*gi.g.nb ? (unsigned) limit : ~0u;
 }
 
 } // namespace
@@ -261,7 +292,7 @@ namespace fteik_capi {
 bool locator_tables_changed()
 {
     gi.ready = gi.off = false;
-    gi.searches = 0;
+    gi.searches = gi.pause = 0;
     return settle_origin_times();
 }
 
@@ -275,7 +306,7 @@ void index_release()
 }
 
 int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
-                 double *objOpt)
+                 double *objOpt, std::vector<int> *redo)
 {
     if (n > kIndexEvents || gi.off || gl.ngrd < 4096 || fteik_k_locate_index_nt(gl.ntf) == 0)
         return 1;
@@ -286,6 +317,7 @@ int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
         if ((size_t) evnmbr[e] > gl.plain.size() ||
             !gl.plain[(size_t) (evnmbr[e] - 1)]) return 1;
     if (!worth_it(n)) { gi.searches++; return 1; }
+    if (n > 1 && gi.pause > 0) { gi.pause--; return 1; }
     if (!gi.ready) {
         if (!build()) return 2;
         if (!gi.ready) return 1;
@@ -314,6 +346,9 @@ int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
         o = ov.data(); w = wv.data(); sk = sv.data();
     }
     hipStream_t s = g_dev.stream;
+    // (of a batch: its share, whatever the batches before it left)
+    const unsigned limit = block_limit(n);
+    const int eb = gi.g.eb, nbatch = (n + eb - 1)/eb;
     bool ok = hipMemcpyAsync(gi.d_obs, o, m*sizeof(float),
                              hipMemcpyHostToDevice, s) == hipSuccess &&
               hipMemcpyAsync(gi.d_wt, w, m*sizeof(float),
@@ -322,21 +357,27 @@ int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
                   == hipSuccess &&
               fteik_k_locate_index_events(&gi.g, &gi.v, n, gl.lntf, gi.d_obs,
                                           gi.d_wt, gi.d_skip, s) == 0;
-    for (int e0 = 0; e0 < n && ok; e0 += gi.g.eb)
-        ok = fteik_k_locate_index_search(&gi.g, &gi.v, e0,
-                                         std::min(gi.g.eb, n - e0),
-                                         std::max(1, g_dev.ncu), s) == 0;
+    for (int q = 0; q < nbatch && ok; q++) {
+        const int m = std::min(eb, n - q*eb);
+        ok = fteik_k_locate_index_search(
+                 &gi.g, &gi.v, q*eb, m,
+                 limit == ~0u ? limit
+                              : (unsigned) ((double) limit*m/n),
+                 gi.v.over + q, std::max(1, g_dev.ncu), s) == 0;
+    }
     ok = ok && fteik_k_locate_index_origin(&gi.g, &gi.v, n, gl.d_tab,
                                            gl.ldgrd, gl.lntf, gi.d_skip,
                                            s) == 0;
-    // keys, then origin times
-    std::vector<unsigned long long> r((size_t) n + ((size_t) n + 1)/2);
+    // keys, then origin times, then the batches given up
+    std::vector<unsigned long long> r(2*(size_t) n);
     ok = ok && d2h(r.data(), gi.v.best, (size_t) n*(sizeof(r[0]) +
-                                                    sizeof(float)));
+                   sizeof(float)) + (size_t) nbatch*sizeof(unsigned));
     if (!ok) return 2;
     gi.through++;
     const float *t0 = (const float *) (r.data() + n);
+    const unsigned *over = (const unsigned *) (t0 + n);
     for (int e = 0; e < n; e++) {
+        if (limit != ~0u && over[e/eb]) { redo->push_back(e); continue; }
         const unsigned bits = (unsigned) (r[(size_t) e] >> 32);
         float obj;
         memcpy(&obj, &bits, sizeof(obj));
@@ -344,6 +385,9 @@ int index_search(int n, const int *evnmbr, int *optIndx, double *t0Opt,
         objOpt[e] = (double) obj;
         t0Opt[e] = (double) t0[e] + gl.tepoch[(size_t) (evnmbr[e] - 1)];
     }
+    // tables or picks that the index is no help with: the bounds cost up to
+    // a tenth of the full search, so look again only now and then
+    if (n > 1 && 2*redo->size() > (size_t) n) gi.pause = 15;
     return 0;
 }
 

@@ -87,16 +87,21 @@ struct LocIndex {
     int eb;
     float* lbs;                    // [ns][eb] bounds of the groups
     int* pair;                     // [ns*eb][2] (group, event) that stay
-    int* npair;                    // their count (8 bytes)
+    int* npair;                    // their count, the blocks' (kLocCounts)
     float* lbc;                    // [ns*eb][64] bounds of their blocks
 };
 constexpr int kLocEv = 8;          // events per group of picks
+// words of LocIndex::npair: the pairs' count, and from word kLocLine on the
+// count of the blocks left, in 64 parts a cache line each (one word for all
+// waves cost 0.45 ms of a search of 4,096 events)
+constexpr int kLocLine = 32, kLocCounts = 65*kLocLine;
 struct LocEvents {
     float *o8, *w8, *h8;           // [n/8][ntf][8] picks, w, sqrt(1/2) w
     float* row;                    // [n][nt][3] the same by event
     float *xn, *kap, *mar;         // [n] 1/sum w, kappa, rounding margin
     unsigned long long* best;      // [n] argmin keys
     float* t0;                     // [n] origin times
+    unsigned* over;                // per batch of events: not 0: given up
 };
 
 // Grid of a ray trace (rays.hip): 2D grids have ny = 1 and is3d = 0.
@@ -252,7 +257,8 @@ int fteik_k_locate_index_events(const fteik::LocIndex* g,
                                 const unsigned char* skip, hipStream_t s);
 int fteik_k_locate_index_search(const fteik::LocIndex* g,
                                 const fteik::LocEvents* v, int e0, int n,
-                                int ncu, hipStream_t s);
+                                unsigned limit, unsigned* over, int ncu,
+                                hipStream_t s);
 int fteik_k_locate_index_origin(const fteik::LocIndex* g,
                                 const fteik::LocEvents* v, int n,
                                 const float* tab, long ldgrd, int lntf,

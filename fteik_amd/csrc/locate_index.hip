@@ -36,6 +36,7 @@
 namespace {
 
 using fteik::LocIndex;
+using fteik::kLocLine;
 
 constexpr int EV = fteik::kLocEv;     // events a thread carries (k_group)
 constexpr float kEps = 1.1920929e-7f; // 2^-23
@@ -377,7 +378,7 @@ __device__ __forceinline__ float misfit(Picks row, float xn,
 // overflow.
 template <int NT>
 __global__ __launch_bounds__(64)
-void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
+void k_children(LocIndex g, fteik::LocEvents v, int e0, int n, unsigned limit)
 {
     // a group's waves adjoin: they read the same blocks, and its pairs adjoin
     // in the list
@@ -389,10 +390,12 @@ void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
     float T[NT], H[NT];
     const int q0 = ((int) blockIdx.x - s*nc)*64, q = q0 + lane;
     unsigned long long low = ~0ull;
+    float keep = 0.0f;
     bool st = false;
     if (q < n) {
         low = best_so_far(v.best + e0 + q);
-        st = stays(g.lbs[(long) s*g.eb + q], keep_norm(low));
+        keep = keep_norm(low);
+        st = stays(g.lbs[(long) s*g.eb + q], keep);
     }
     unsigned long long m = __ballot(st);
     if (m == 0) return;
@@ -402,7 +405,7 @@ void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
         T[i] = g.rep[(long) min(i, g.ntf - 1)*g.nb + cb];
         H[i] = g.h[(long) min(i, g.ntf - 1)*g.nb + cb];
     }
-    int at = 0;
+    int at = 0, left = 0;
     if (lane == 0) at = atomicAdd(g.npair, __popcll(m));
     at = __builtin_amdgcn_readfirstlane(at);
     for (; m; m &= m - 1, at++) {
@@ -423,9 +426,18 @@ void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
             g.pair[2*(long) at] = s;
             g.pair[2*(long) at + 1] = e;
         }
-        g.lbc[(long) at*64 + lane] = b >= 0
-            ? low_norm(ob, 2.0f*s2, v.kap[e], v.mar[e]) : __builtin_inff();
+        const float lb = b >= 0 ? low_norm(ob, 2.0f*s2, v.kap[e], v.mar[e])
+                                : __builtin_inff();
+        g.lbc[(long) at*64 + lane] = lb;
+        if (limit != ~0u) {
+            // (by the minimum at the wave's start: rather too many)
+            const float kp = __uint_as_float((unsigned)
+                __builtin_amdgcn_readlane((int) __float_as_uint(keep), w));
+            left += __popcll(__ballot(b >= 0 && stays(lb, kp)));
+        }
     }
+    if (limit != ~0u && lane == 0)
+        atomicAdd(g.npair + (1 + (blockIdx.x & 63))*kLocLine, left);
 }
 
 // Cells of the blocks that stay: one wave per (group, event) of the list, a
@@ -437,11 +449,23 @@ void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
 //
 // With few events the list is short: `sl` waves (a power of two) share a
 // pair's blocks.
+//
+// With more than `limit` blocks left in the batch (~0: no limit) none is
+// evaluated and `over` is set: the caller searches in full.
 template <int NT>
 __global__ __launch_bounds__(64)
-void k_cells(LocIndex g, fteik::LocEvents v, int sl)
+void k_cells(LocIndex g, fteik::LocEvents v, int sl, unsigned limit,
+             unsigned* __restrict__ over)
 {
     const int lane = threadIdx.x;
+    if (limit != ~0u) {
+        unsigned left = (unsigned) g.npair[(1 + lane)*kLocLine];
+        for (int off = 32; off > 0; off >>= 1)
+            left += __shfl_xor(left, off, 64);
+        const bool up = left > limit;
+        if (blockIdx.x == 0 && lane == 0) *over = up;
+        if (up) return;
+    }
     const int np = *g.npair*sl, per = (np + 7)/8, xcd = blockIdx.x & 7;
     const int p1 = min(np, (xcd + 1)*per);
     for (int ps = xcd*per + ((int) blockIdx.x >> 3); ps < p1;
@@ -544,19 +568,23 @@ int fteik_k_locate_index_events(const LocIndex* g, const fteik::LocEvents* v,
 }
 
 int fteik_k_locate_index_search(const LocIndex* g, const fteik::LocEvents* v,
-                                int e0, int n, int ncu, hipStream_t s)
+                                int e0, int n, unsigned limit,
+                                unsigned* over, int ncu, hipStream_t s)
 {
     if (e0 % EV != 0 || n < 1 || n > g->eb) return 2;
-    if (fteik_k_fill_u64((unsigned long long*) g->npair, 1, 0ull, s)) return 1;
+    if (fteik_k_fill_u64((unsigned long long*) g->npair, fteik::kLocCounts/2,
+                         0ull, s)) return 1;
     hipLaunchKernelGGL(k_group, dim3((g->ns + 63)/64, (n + EV - 1)/EV),
                        dim3(64), 0, s, *g, *v, e0, n);
     const dim3 gc((unsigned) g->ns*(unsigned) ((n + 63)/64));
     // waves of k_cells: what the registers of NT times leave resident
 #define LI(N) case N: \
-        hipLaunchKernelGGL(k_children<N>, gc, dim3(64), 0, s, *g, *v, e0, n); \
+        hipLaunchKernelGGL(k_children<N>, gc, dim3(64), 0, s, *g, *v, e0, n, \
+                           limit); \
         hipLaunchKernelGGL(k_cells<N>, dim3((N <= 32 ? 32 : N <= 64 ? 20 : 16) \
                                             *((ncu + 7)/8*8)), \
-                           dim3(64), 0, s, *g, *v, n <= 64 ? 8 : 1); \
+                           dim3(64), 0, s, *g, *v, n <= 64 ? 8 : 1, limit, \
+                           over); \
         break;
     switch (g->nt) {
         LI(8) LI(16) LI(24) LI(32) LI(40) LI(48) LI(64) LI(80) LI(96)

@@ -176,3 +176,35 @@ def test_origin_times_carry_over_from_the_old_tables(change):
     assert loc.locateEvent(1) == ref.locate(1, accumulate_t0=True,
                                             pad_argmin=True)
     loc.finalize()
+
+
+@pytest.mark.parametrize("kind,shape", [
+    ("smooth", (81, 161, 161)), ("noise", (60, 60, 70))])
+def test_large_calls_equal_full_search(kind, shape):
+    """8,192 events through the index against a call of 8,193, which is
+    searched in full: smooth tables, whose work space takes the events in two
+    batches, and tables without structure, whose batch is given up after the
+    bounds and searched in full (and so are the next calls)."""
+    print("case:", kind, shape, flush=True)
+    rng = np.random.default_rng(31)
+    ntf, n = 8, 8193
+    tables = _tables(rng, ntf, *shape) if kind == "smooth" else \
+        rng.uniform(0, 9, (ntf, int(np.prod(shape)))).astype(np.float32)
+    f = lib().fteik_k_locate_index_searches
+    f.restype = ctypes.c_int
+    loc = fa.Locator(n, ntf, tables.shape[1])
+    loc.setReferenceCompatibility(0)
+    for k in range(ntf):
+        loc.setTravelTimeField(k + 1, tables[k])
+    for e, (k, t, w) in enumerate(_events(rng, tables, n, 0.1)):
+        loc.setObservation(e + 1, k, t, w)
+    ev = np.arange(1, n + 1)
+    full = loc.locateEvents(ev)
+    assert f() == 0
+    for calls in (1, 2):
+        got = loc.locateEvents(ev[:-1])
+        assert f() == (calls if kind == "smooth" else 1)
+        for a, b in zip(got, full):
+            np.testing.assert_array_equal(a, b[:-1])
+    loc.setReferenceCompatibility(1)
+    loc.finalize()
