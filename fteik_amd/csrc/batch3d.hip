@@ -52,7 +52,7 @@ void batch_sweep_kernel(const BatchGrid* __restrict__ grids,
     a.mbx = a.mby = nullptr; a.mbnt = 0;
     a.colmod = nullptr; a.plan = nullptr;
     a.stamp = nullptr; a.lastchg = nullptr;
-    a.count = 0; a.code = 0; a.mbBytes = 0; a.runs = nullptr;
+    a.count = 0; a.code = 0; a.load = 0; a.mbBytes = 0; a.runs = nullptr;
     if (a.fz0 > a.fz1 || a.fx0 > a.fx1 || a.fy0 > a.fy1) {
         if (threadIdx.x == 0)
             __hip_atomic_store(flags + m.flag, (serial << 32) | 0xffffffffull,
@@ -96,7 +96,7 @@ __global__ void batch_mb_args_kernel(const BatchGrid* __restrict__ grids,
                                      int bx, int by,
                                      unsigned long long serial,
                                      int* __restrict__ err, int fp32,
-                                     int track, unsigned count,
+                                     int track, unsigned count, int load,
                                      SweepArgs<R>* __restrict__ args)
 {
     const int i = blockIdx.x*blockDim.x + threadIdx.x;
@@ -124,7 +124,7 @@ __global__ void batch_mb_args_kernel(const BatchGrid* __restrict__ grids,
     a.pserial = 0; a.par = 0; a.psz = a.psx = a.psy = 0;
     a.stamp = count ? g.stamp : nullptr;
     a.lastchg = g.lastchg;
-    a.count = count; a.code = stamp_code(count);
+    a.count = count; a.code = stamp_code(count); a.load = load;
     a.mbBytes = g.mbBytes; a.runs = nullptr;
     args[i] = a;
 }
@@ -290,7 +290,8 @@ extern "C" int fteik_k_batch_mb_sweep(const BatchGrid* grids, int ngrids,
                                       int sweep, int linit,
                                       unsigned long long serial,
                                       int* err, int fp32, int track,
-                                      int chunk, unsigned count, int cube,
+                                      int chunk, unsigned count, int load,
+                                      int cube,
                                       void* argbuf, hipStream_t stream)
 {
     if (tile < 0 || tile >= kNumTiles || kTiles[tile].mode == 0 || nwg < 0 ||
@@ -313,12 +314,12 @@ extern "C" int fteik_k_batch_mb_sweep(const BatchGrid* grids, int ngrids,
         hipLaunchKernelGGL(batch_mb_args_kernel<float>, dim3((ngrids + 63)/64),
                            dim3(64), 0, stream, grids, ngrids, sweep, linit,
                            ts.bx, ts.by, serial, err, fp32, track, count,
-                           (SweepArgs<float>*) argbuf);
+                           load, (SweepArgs<float>*) argbuf);
     else
         hipLaunchKernelGGL(batch_mb_args_kernel<double>,
                            dim3((ngrids + 63)/64), dim3(64), 0, stream, grids,
                            ngrids, sweep, linit, ts.bx, ts.by, serial, err,
-                           fp32, track, count,
+                           fp32, track, count, load,
                            (SweepArgs<double>*) argbuf);
     void* args[] = {&argbuf, (void*) &map};
     hipError_t e = hipLaunchKernel(fn, dim3(nwg),

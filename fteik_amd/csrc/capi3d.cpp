@@ -136,8 +136,8 @@ bool reset_skipping(SweepLaunch &L)
         L.lastchg = g3.d_lastchg;
         g3.count = 0;
         return hipMemsetAsync(g3.d_stamp, 0, nb, g_dev.stream) == hipSuccess
-            && hipMemsetAsync(g3.d_lastchg, 0, sizeof(unsigned),
-                              g_dev.stream) == hipSuccess;
+            && hipMemsetAsync(g3.d_lastchg, 0, fteik_k_record_words()*
+                              sizeof(unsigned), g_dev.stream) == hipSuccess;
     }
     L.colmod = g3.d_colmod; L.lastproc = g3.d_lastproc; L.plan = g3.d_plan;
     return fteik_k_fill_u64(g3.d_colmod, (long) g3.nx*g3.ny, 1ull,
@@ -362,7 +362,8 @@ void fteik_solver3d_initialize(int nz, int nx, int ny, double z0, double x0,
     if (g3.chunkFits) {
         const size_t rw = fteik_k_run_words(nx, ny);
         if (dalloc(&g3.d_stamp, fteik_k_stamp_bytes(ngrd)) &&
-            dalloc(&g3.d_lastchg, 1) && dalloc(&g3.d_runs, rw)) {
+            dalloc(&g3.d_lastchg, fteik_k_record_words()) &&
+            dalloc(&g3.d_runs, rw)) {
             hipMemsetAsync(g3.d_runs, 0, rw*sizeof(unsigned long long),
                            g_dev.stream);
         } else {
@@ -414,7 +415,7 @@ void fteik_solver3d_initialize(int nz, int nx, int ny, double z0, double x0,
     g3.cooperative = first >= 0;
     g3.tile = g3.tile32 = first >= 0 ? first : 0;
     // The iteration sweeps run on chunked tiles, which skip by node and not
-    // by tile: a solve of 33 x 29 x 31 nodes 2.2 -> 1.6 ms, 101^3 6.3 -> 5.3
+    // by tile: a solve of 33 x 29 x 31 nodes 2.2 -> 1.6 ms, 101^3 6.3 -> 5.1
     // ms, 257^3 104 -> 84 ms, 131 x 190 x 157 in mixed precision 60 -> 49 ms
     // (streamed tiles with tile skipping before).  The initialization sweeps
     // keep the tile above.

@@ -50,12 +50,12 @@ struct Batch3D {
     int *d_mbmap = nullptr;
     char *d_mbargs = nullptr;
     // change record of the chunked tiles' iteration sweeps: the grids' bytes
-    // one after another, then a word per grid (last changing sweep); count:
-    // sweeps recorded
+    // one after another after the grids' words; count: sweeps recorded
     unsigned char *d_stamp = nullptr;
     size_t stampCap = 0;
     unsigned count = 0;
     bool cube = false;               // every grid has equal spacings
+    int load = 0;                    // how full the sweeps keep the CUs
     int *d_err = nullptr;
     double *d_maxdelta = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -129,14 +129,25 @@ bool batch_prepare(const char *who)
                            g_dev.stream);
         }
     }
+    double nodes = 0.0;
+    int levels = 1;
+    for (const BGrid &x : gb.g) {
+        nodes += (double) x.nz*x.nx*x.ny;
+        levels = std::max(levels, x.nz + x.nx + x.ny);
+    }
+    const double perCU = nodes/levels/(g_dev.ncu > 0 ? g_dev.ncu : 256);
     gb.chunked = gb.chunk && edge;
+    // (in 64ths of the chunks, see batch_share: 23 of 16 grids of 64 .. 192
+    // nodes per axis, 10 where 128 nodes per level and CU leave the chains)
+    gb.load = (int) std::min(64.0*perCU/800.0, 64.0);
     for (const BGrid &x : gb.g)
         gb.chunked = gb.chunked && fteik_k_chunk_fits(
             x.nz, x.nx, x.ny, sizeof(unsigned long long)*
             (edge_words(x, false) + edge_words(x, true)));
     // change record (chunked tiles): words first, then each grid's bytes;
     // where it finds no memory the streamed tiles run every sweep
-    size_t stoff = ((size_t) ng*sizeof(unsigned) + 255)/256*256;
+    const size_t rec = (size_t) fteik_k_record_words();
+    size_t stoff = (ng*rec*sizeof(unsigned) + 255)/256*256;
     if (gb.chunked) {
         size_t bytes = stoff;
         for (const BGrid &x : gb.g)
@@ -184,7 +195,7 @@ bool batch_prepare(const char *who)
         d.lastchg = nullptr;
         if (gb.d_stamp) {
             d.stamp = gb.d_stamp + stoff + fteik_k_stamp_offset();
-            d.lastchg = (unsigned *) gb.d_stamp + i;
+            d.lastchg = (unsigned *) gb.d_stamp + rec*i;
             stoff += fteik_k_stamp_bytes((long) x.nz*x.nx*x.ny);
         }
         d.nz = x.nz; d.nx = x.nx; d.ny = x.ny;
@@ -269,7 +280,7 @@ bool batch_sweep(int sweep, bool linit, bool fp32, bool track)
                                               fp32 ? 1 : 0, track ? 1 : 0,
                                               gb.chunked ? 1 : 0,
                                               (!linit && gb.chunked)
-                                              ? ++gb.count : 0,
+                                              ? ++gb.count : 0, gb.load,
                                               gb.cube ? 1 : 0,
                                               gb.d_mbargs, g_dev.stream);
         if (rc != 0) msg("fteik_batch3d_solve: sweep launch failed (%d)", rc);

@@ -45,7 +45,7 @@ struct SweepLaunch {
     unsigned long long* prog;
     // chunk: iteration sweeps with the chunked tiles (sweep_chunk.h); their
     // change record (fteik_k_stamp_bytes bytes; null: no chunk skipping),
-    // last changing sweep, number of this iteration sweep, and the tiles'
+    // its fteik_k_record_words words, number of this iteration sweep, and the tiles'
     // run words (fteik_k_run_words, zeroed once; serials only grow)
     int chunk;
     unsigned long long* runs;
@@ -139,16 +139,19 @@ int fteik_k_batch_mb_sweep(const fteik::BatchGrid* grids, int ngrids,
                            const int* map, int nwg, int tile, int sweep,
                            int linit, unsigned long long serial, int* err,
                            int fp32, int track, int chunk, unsigned count,
-                           int cube, void* argbuf, hipStream_t stream);
+                           int load, int cube, void* argbuf,
+                           hipStream_t stream);
 // sweep_chunk.hip: the chunked tiles' kernels (count: number of the sweep
-// in the record, 0 without one; cube: every grid has equal spacings),
-// whether a grid can use them (mbBytes: of its edge-major mailboxes), the
-// bytes of its change record and the words of its tiles' runs
+// in the record, 0 without one; cube: every grid has equal spacings; a
+// batch's load: see batch_share), whether a grid can use them
+// (mbBytes: of its edge-major mailboxes), the bytes and words of its change
+// record and the words of its tiles' runs
 int fteik_k_chunk_fits(int nz, int nx, int ny, size_t mbBytes);
 size_t fteik_k_run_words(int nx, int ny);
 const void* fteik_k_chunk_fn(int fp32, unsigned count, int batch, int cube);
 size_t fteik_k_stamp_bytes(long ngrd);
 long fteik_k_stamp_offset(void);
+int fteik_k_record_words(void);
 // sweep3d.hip
 int fteik_k_sweep3d(const fteik::SweepLaunch* L, int sweep, int linit,
                     hipStream_t stream);

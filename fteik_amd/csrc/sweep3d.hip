@@ -356,7 +356,7 @@ static int launch_sweep_t(const SweepLaunch& L, int sweep, bool linit,
     a.mbx = L.mbx; a.mby = L.mby; a.mbnt = L.mbnt;
     a.colmod = nullptr; a.plan = nullptr;
     a.stamp = nullptr; a.lastchg = nullptr;
-    a.count = 0; a.code = 0; a.mbBytes = 0; a.runs = nullptr;
+    a.count = 0; a.code = 0; a.load = 0; a.mbBytes = 0; a.runs = nullptr;
     if (a.fz0 > a.fz1 || a.fx0 > a.fx1 || a.fy0 > a.fy1) return 0;
     if (L.schedule == 1) {
         const int nlev = (a.fz1 + a.fx1 + a.fy1) - (a.fz0 + a.fx0 + a.fy0) + 1;

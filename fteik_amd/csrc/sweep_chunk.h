@@ -32,7 +32,8 @@
 // bytes per column is read.  Mailbox entries carry the dirty bit, and a
 // skipped chunk posts entries without a value: a reader that needs one
 // takes it from the field, which this launch does not change there.  The
-// first eight sweeps of a record (RECORD without SKIP) compute every chunk.
+// first eight sweeps of a record (RECORD without SKIP) compute every chunk,
+// and so do later ones where much is dirty (sweep_is_busy).
 // Measured (one wave, batches): 16 grids of 64 .. 192 nodes per axis, 12
 // iterations, 98 -> 29 ms (streamed tiles before); 48 tables of 81 x 161 x
 // 161, 2 iterations, 50 -> 31 ms; 8 of the 16 grids in mixed precision 84 ->
@@ -40,8 +41,8 @@
 // is the issue rate of FP64 instructions in its active chunks and, where
 // little is left to do, a mailbox round trip per skipped chunk.
 // Three waves, single grids: a level of a lone tile 0.48 us (streamed tiles
-// 0.68), a dense 257^3 sweep 625 us (735), its solve of 19 iterations 104 ->
-// 84 ms, 101^3 with 2 iterations 6.3 -> 5.3 ms.  A dense sweep is its chain
+// 0.68), a dense 257^3 sweep 615 us (725), its solve of 19 iterations 104 ->
+// 84 ms, 101^3 with 2 iterations 6.3 -> 5.1 ms.  A dense sweep is its chain
 // of chunks (193 at 1.9 us) and a hop of 4 us, a chunk and the mailbox, for
 // each of 62 tiles from corner to corner; a sweep with nothing left to do is
 // the hops.
@@ -187,6 +188,15 @@ __host__ __device__ inline bool chunk_fits(long nz, long nx, long ny,
            nz < (1 << 17) && nx < (1 << 20) && ny < (1 << 20);
 }
 
+// Words of a grid's record: the last changing sweep, then the number of
+// chunks that a sweep changed, for the last sixteen sweeps.
+constexpr int kRecordWords = 32;
+template <typename R>
+__device__ __forceinline__ unsigned* changed_chunks(const SweepArgs<R>& a,
+                                                    unsigned count)
+{
+    return a.lastchg + 1 + (count & 15u);
+}
 // One tile as a lane sees it: geometry, addresses, and the loads and stores
 // of a chunk.  Fields that a wave does not use cost it nothing.
 template <typename R>
@@ -525,10 +535,12 @@ struct ChunkTile {
         #pragma unroll
         for (int i = 0; i < 4; i++) out[i] = p[18*i];
     }
+    // nchg: chunks that changed (uniform, with RECORD)
     template <bool RECORD>
     __device__ void store(int t0, const R (&old)[4], const R (&out)[4],
-                          R& dmax, bool& changed) const
+                          R& dmax, int& nchg) const
     {
+        bool changed = false;
         #pragma unroll
         for (int i = 0; i < 4; i++) {
             const bool ch = out[i] != old[i];
@@ -538,18 +550,21 @@ struct ChunkTile {
             changed = changed || ch;
             dmax = ch ? rmax(dmax, old[i] - out[i]) : dmax;
         }
+        if (RECORD) nchg += __ballot(changed) != 0 ? 1 : 0;
     }
     template <bool RECORD>
-    __device__ void finish(R dmax, bool changed) const
+    __device__ void finish(R dmax, int nchg) const
     {
         if (a.maxdelta && dmax > R(0)) {
             const double dd = (double) dmax;
             atomicMax((unsigned long long*) a.maxdelta,
                       (unsigned long long) __double_as_longlong(dd));
         }
-        if (RECORD && __ballot(changed) != 0 && lane == 0)
+        if (RECORD && nchg > 0 && lane == 0) {
             __hip_atomic_store(a.lastchg, a.count, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
+            atomicAdd(changed_chunks(a, a.count), (unsigned) nchg);
+        }
     }
 };
 
@@ -561,6 +576,53 @@ __device__ __forceinline__ bool sweep_is_clean(const SweepArgs<R>& a)
 {
     return __hip_atomic_load(a.lastchg, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT) + 7u < a.count;
+}
+
+// A chunk that looks for dirty nodes and has some takes longer than one that
+// is computed in any case (three waves, lone tile: 2.7 against 1.95 us; one
+// wave: a tenth longer), and the more tiles a sweep has to cross, the less it
+// gains from a clean chunk: it waits for the tiles that have work.  So a sweep
+// computes every chunk where the last seven changed more than `share` (64ths)
+// of them, all seven together: about 1.2 to 1.5 times the chunks that have a
+// dirty node, more on grids of few tiles, whose changes stay in one place.
+// Every tile of a grid decides alike, from launches before this one.
+template <typename R>
+__device__ __forceinline__ bool sweep_is_busy(const SweepArgs<R>& a, int share)
+{
+    unsigned n = 0;
+    #pragma unroll
+    for (unsigned k = 1; k <= 7; k++) n += *changed_chunks(a, a.count - k);
+    const int chunks = a.nbx*a.nby*((a.fz1 - a.fz0 + 2*CB)/CK + 1);
+    return (long) n*64 > (long) chunks*share;
+}
+// Single grids.  Where a sweep that skips is as fast as one that computes
+// every chunk, smooth random velocities: 25 % of the chunks at 33^3 nodes (6
+// tiles to cross), 7 % at 129^3 (30), 5 % at 257^3 (62).  129 x 257 x 257
+// nodes, 8 iterations, most chunks dirty in six of them: 45.0 ms skipping in
+// all, 36.5 with this line (streamed tiles 39.9).
+template <typename R>
+__device__ __forceinline__ int single_share(const SweepArgs<R>& a)
+{
+    return max(4, 96/max(a.nbx + a.nby - 2, 2));
+}
+// Batches.  a.load: where the SIMDs have their waves of other tiles every
+// clean chunk counts.  6 grids of 128^3 nodes, rough velocities, 12
+// iterations: 47.3 ms skipping in all, 41 with this line (streamed 44.5); 16
+// smooth ones of 64 .. 192 nodes per axis 34.9 and 34.7.  Grids of few tiles
+// never compute every chunk: 256 of 200 x 20 x 20, 32.6 ms skipping, 36.5
+// with a line of 3/4 of the chunks.
+template <typename R>
+__device__ __forceinline__ int batch_share(const SweepArgs<R>& a)
+{
+    const int hops = a.nbx + a.nby - 2;
+    return hops < 6 ? 7*64
+                    : max(max(4, a.load), max(192/hops, 1536/(hops*hops)));
+}
+// The grid's first tile clears the next sweep's count.
+template <typename R>
+__device__ __forceinline__ void clear_count(const SweepArgs<R>& a, int wg)
+{
+    if (wg == 0 && threadIdx.x == 0) *changed_chunks(a, a.count + 1) = 0;
 }
 
 template <typename R, bool CUBE>
@@ -655,6 +717,8 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
     const int lane = threadIdx.x;
     const ChunkTile<R> T(a, wg, lane, RECORD);
     if (T.empty() || (SKIP && sweep_is_clean(a))) return;
+    // (one body for both: the two side by side spill registers)
+    const bool skip = SKIP && !sweep_is_busy(a, batch_share(a));
     const Consts<R> c = chunk_consts<R, CUBE>(a);
     // What the chunk before left: prevDirty, its steps 1..3 hold a dirty
     // node (own, halo); loaded: its times, cells and halo are in LDS.
@@ -666,11 +730,11 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
     R tnx[4], cnx[CNC];
     unsigned stn = 0;
     R dmax = R(0);
-    bool changed = false;
+    int nchg = 0;
     int half = 0;                       // ring and cell half of the chunk
-    if (SKIP) stn = T.load_stamp(T.tlo - CK);
+    if (skip) stn = T.load_stamp(T.tlo - CK);
     T.load_entries(T.tlo - CK, e0, e1);
-    T.load_direct(T.tlo - CK, SKIP, d0, d1, b0, b1);
+    T.load_direct(T.tlo - CK, skip, d0, d1, b0, b1);
     for (int t0 = T.tlo - CK; t0 <= T.thi; t0 += CK, half ^= 4) {
         const bool more = t0 + CK <= T.thi;
         // ---- the upwind neighbours' chunk
@@ -688,9 +752,9 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
         // ---- dirty nodes among those the chunk reads: steps t0 - 3 .. t0
         // + 2 of the own and the halo columns
         unsigned own = 0;
-        bool active = !SKIP && t0 >= T.tlo;
+        bool active = !skip && t0 >= T.tlo;
         bool nextDirty = false;
-        if (SKIP) {
+        if (skip) {
             own = T.own_dirty(t0, stn);
             if (more) stn = T.load_stamp(t0 + CK);
             bool hd, cd;
@@ -746,14 +810,14 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
                 T, c, t0, rp, rc, ch, co, tbuf, past, [&]() {
                     if (more) {
                         T.load_entries(t0 + CK, e0, e1);
-                        T.load_direct(t0 + CK, SKIP, d0, d1, b0, b1);
+                        T.load_direct(t0 + CK, skip, d0, d1, b0, b1);
                     }
                 });
             own |= chg;
-            if (SKIP) nextDirty = nextDirty || (chg & 14u);
+            if (skip) nextDirty = nextDirty || (chg & 14u);
         } else if (more) {
             T.load_entries(t0 + CK, e0, e1);
-            T.load_direct(t0 + CK, SKIP, d0, d1, b0, b1);
+            T.load_direct(t0 + CK, skip, d0, d1, b0, b1);
         }
         if (t0 >= T.tlo)
             T.post(t0, active, rc, SKIP ? (unsigned) __shfl((int) own,
@@ -767,13 +831,13 @@ __device__ __forceinline__ void chunk_body(const SweepArgs<R>& a, const int wg)
                 T.park_t(tbuf, tnx);
                 T.park_c(ch, cnx);
             }
-            T.template store<RECORD>(t0, tw, out, dmax, changed);
+            T.template store<RECORD>(t0, tw, out, dmax, nchg);
             wave_lds_fence();
         }
         loaded = active;
-        prevDirty = SKIP && __ballot(nextDirty) != 0;
+        prevDirty = skip && __ballot(nextDirty) != 0;
     }
-    T.template finish<RECORD>(dmax, changed);
+    T.template finish<RECORD>(dmax, nchg);
 }
 
 // -------------------------------------------------------- three waves
@@ -806,22 +870,44 @@ constexpr int kRunStride = 16;          // words
 constexpr int kMaxDirt = 1024;          // chunks of s_dirt: nz up to 4000
 constexpr int kNews = 64;
 enum : int { kSkipClean = 0, kSkipDirty = 1, kCompute = 2 };
+// A thread's index that the compiler does not know to be the same in the two
+// bodies of a kernel that chooses between them: what it could form from it
+// once for both would hold registers through either (20 VGPRs spilled).
+__device__ __forceinline__ int own_index(int i)
+{
+    asm volatile("" : "+v"(i));
+    return i;
+}
+
+template <typename R>
+struct Chunk3Lds {
+    R ring[12*CROW], cbuf[12*CROW], tbuf[3*CK*CTROW];
+    unsigned char own[3][64], chg[3][64];
+    // announcement k in slot k mod kNews: what becomes of the next chunks,
+    // kSkipClean (nothing dirty of its own), kSkipDirty (see own) or
+    // kCompute, and, from bit 2 on, how many they are; the chunk it starts
+    // at; any, per part: whether the chunk changed a node on its steps 1..3
+    int news[kNews], start[kNews], any[3];
+    unsigned char dirt[kMaxDirt];
+    int load, comp, store, abort;
+};
 template <typename R, bool SKIP, bool RECORD, bool CUBE>
 __device__ __forceinline__ void chunk3_body(const SweepArgs<R>& a,
-                                            const int wg)
+                                            const int wg, Chunk3Lds<R>& lds)
 {
-    __shared__ R ring[12*CROW];
-    __shared__ R cbuf[12*CROW];
-    __shared__ R tbuf[3*CK*CTROW];
-    __shared__ unsigned char s_own[3][64], s_chg[3][64];
-    // announcement k in slot k mod kNews: what becomes of the next chunks,
-    // kSkipClean (nothing dirty of its own), kSkipDirty (see s_own) or
-    // kCompute, and, from bit 2 on, how many they are; the chunk it starts
-    // at; s_any, per part: whether the chunk changed a node on its steps 1..3
-    __shared__ int s_news[kNews], s_start[kNews], s_any[3];
-    __shared__ unsigned char s_dirt[SKIP ? kMaxDirt : 1];
-    __shared__ int g_load, g_comp, g_store, s_abort;
-    const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
+    R* const ring = lds.ring;
+    R* const cbuf = lds.cbuf;
+    R* const tbuf = lds.tbuf;
+    unsigned char (*const s_own)[64] = lds.own;
+    unsigned char (*const s_chg)[64] = lds.chg;
+    int* const s_news = lds.news;
+    int* const s_start = lds.start;
+    int* const s_any = lds.any;
+    unsigned char* const s_dirt = lds.dirt;
+    int &g_load = lds.load, &g_comp = lds.comp, &g_store = lds.store,
+        &s_abort = lds.abort;
+    const int thread = own_index(threadIdx.x);
+    const int lane = thread & 63, role = thread >> 6;
     const ChunkTile<R> T(a, wg, lane, RECORD);
     if (T.empty() || (SKIP && sweep_is_clean(a))) return;     // uniform
     if (threadIdx.x == 0) g_load = g_comp = g_store = s_abort = 0;
@@ -1134,7 +1220,7 @@ __device__ __forceinline__ void chunk3_body(const SweepArgs<R>& a,
     } else {
         // ---------------------------------------------------------- store
         R dmax = R(0);
-        bool changed = false;
+        int nchg = 0;
         int part = 0, avail = 0;
         int first = -1;           // of the clean chunks not yet posted
         for (int g = 0, k = 0; g < ng; k++) {
@@ -1172,10 +1258,10 @@ __device__ __forceinline__ void chunk3_body(const SweepArgs<R>& a,
                 T.collect(rc, out);
             }
             done(&g_store, ++g);
-            if (act) T.template store<RECORD>(t0, old, out, dmax, changed);
+            if (act) T.template store<RECORD>(t0, old, out, dmax, nchg);
             part = part == 2 ? 0 : part + 1;
         }
-        T.template finish<RECORD>(dmax, changed);
+        T.template finish<RECORD>(dmax, nchg);
     }
 }
 

@@ -13,9 +13,14 @@ __global__ __launch_bounds__(192)
 __attribute__((amdgpu_waves_per_eu(3)))
 void sweep3d_chunk_kernel(SweepArgs<R> a)
 {
+    __shared__ Chunk3Lds<R> lds;
     const int wg = tile_of_rank((int) blockIdx.x, a.nbx, a.nby);
     if (wg < 0) return;
-    chunk3_body<R, SKIP, RECORD, CUBE>(a, wg);
+    if (RECORD) clear_count(a, wg);
+    if (SKIP && !sweep_is_busy(a, single_share(a)))
+        chunk3_body<R, true, true, CUBE>(a, wg, lds);
+    else
+        chunk3_body<R, false, RECORD, CUBE>(a, wg, lds);
 }
 
 // Workgroup w sweeps map entry (grid, tile); args[g]: grid g's sweep
@@ -33,10 +38,13 @@ void batch_chunk_kernel(const SweepArgs<R>* __restrict__ args,
 #else   // the host pass only parses the kernel
     const SweepArgs<R> a = args[map[2*blockIdx.x]];
 #endif
-    chunk_body<R, SKIP, RECORD, CUBE>(a, map[2*blockIdx.x + 1]);
+    const int wg = map[2*blockIdx.x + 1];
+    if (RECORD) clear_count(a, wg);
+    chunk_body<R, SKIP, RECORD, CUBE>(a, wg);
 }
 
-// kind 0: every chunk; 1: every chunk, changes recorded; 2: skipping
+// kind 0: every chunk; 1: every chunk, changes recorded; 2: skipping where few
+// chunks are dirty, else as 1
 template <typename R, bool CUBE>
 static const void* chunk_fn(int kind, bool batch)
 {
@@ -79,3 +87,4 @@ extern "C" size_t fteik_k_stamp_bytes(long ngrd)
 }
 
 extern "C" long fteik_k_stamp_offset(void) { return kStampPad; }
+extern "C" int fteik_k_record_words(void) { return kRecordWords; }

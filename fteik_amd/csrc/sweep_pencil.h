@@ -162,13 +162,15 @@ struct SweepArgs {
     int psz, psx, psy;
     // Chunked tiles with skipping (sweep_chunk.h; null: off):
     //   stamp[node]   number (stamp_code) of the sweep that changed it last
-    //   lastchg       number of the last sweep that changed anything
+    //   lastchg       number of the last sweep that changed anything; after
+    //                 it how much each of the last sweeps changed
     //   count, code   number of this sweep (1: the solve's first iteration
     //                 sweep) and its stamp code
     unsigned char* stamp;
     unsigned* lastchg;
     unsigned count;
     int code;
+    int load;                    // of a batch (batch_share)
     unsigned mbBytes;            // of mbx and, after it, mby
     unsigned long long* runs;    // run words of a single sweep's tiles
 };

@@ -125,3 +125,47 @@ def test_chunked_batch(cube, precision):
         if precision == 0:
             np.testing.assert_array_equal(
                 fields[0][i], _oracle(models[i], *c[:4], srcs[i], nsweep))
+
+
+def _serpentine(nz, nx, ny):
+    """Fast corridors along x, joined at alternate ends, between walls of 1
+    m/s: with sources at the first corridor's end the front passes a few bends
+    an iteration."""
+    v = np.ones((ny - 1, nx - 1, nz - 1))
+    v[::2] = 5000.0
+    v[1::4, -1] = 5000.0
+    v[3::4, 0] = 5000.0
+    return v.ravel()
+
+
+SERPENTINE = (3, 10, 260)
+SOURCE = (5.0, 15.0, 5.0)
+D = (10.0, 10.0, 10.0)
+
+
+def test_more_sweeps_than_the_record_has_numbers():
+    """The change record numbers sweeps modulo 255: a field that still changes
+    in every iteration from the 8th to the 40th (sweeps 57 to 320)."""
+    nz, nx, ny = SERPENTINE
+    vel = _serpentine(*SERPENTINE)
+    print("case: serpentine", SERPENTINE, flush=True)
+    L, ierr = lib(), c_int(1)
+    L.fteik_solver3d_initialize(nz, nx, ny, 0.0, 0.0, 0.0, *D, 40, 3.0, 0.0,
+                                0, byref(ierr))
+    assert ierr.value == 0
+    L.fteik_solver3d_setVelocityModel64f(vel.size, _d(vel), byref(ierr))
+    assert ierr.value == 0
+    s = [np.array([a]) for a in SOURCE]
+    L.fteik_solver3d_setSources64f(1, *[_d(a) for a in s], byref(ierr))
+    last = None
+    for nsweep in (31, 32, 33, 40):
+        L.fteik_solver3d_setNumberOfSweeps(nsweep, byref(ierr))
+        L.fteik_solver3d_solveSourceLSM(1, byref(ierr))
+        assert ierr.value == 0
+        tt = np.zeros(nz * nx * ny)
+        L.fteik_solver3d_getTravelTimeField64f(tt.size, 0, _d(tt),
+                                               byref(ierr))
+        np.testing.assert_array_equal(
+            tt, _oracle(vel, nz, nx, ny, D, SOURCE, nsweep))
+        assert last is None or np.any(tt != last)
+        last = tt
