@@ -129,6 +129,13 @@ bool batch_prepare(const char *who)
                            g_dev.stream);
         }
     }
+    // Chunked tiles, of one wave each in a batch, wait for their own stores:
+    // they need others beside them.  Nodes per level of the sweeps (the most
+    // levels of a grid) at which they are as fast as the streamed tiles: about
+    // 24,000.  2 grids of 64 .. 128 nodes per axis, 6 iterations (8,000):
+    // 16.3 ms, streamed 14.1; 4 of 118 x 176 x 187, 2 iterations (26,400):
+    // 12.0, streamed 12.9; 16 flat ones of 8 x 160 x 160 (10,000): 9.2 and
+    // 7.7.
     double nodes = 0.0;
     int levels = 1;
     for (const BGrid &x : gb.g) {
@@ -136,7 +143,7 @@ bool batch_prepare(const char *who)
         levels = std::max(levels, x.nz + x.nx + x.ny);
     }
     const double perCU = nodes/levels/(g_dev.ncu > 0 ? g_dev.ncu : 256);
-    gb.chunked = gb.chunk && edge;
+    gb.chunked = gb.chunk && edge && perCU >= 96.0;
     // (in 64ths of the chunks, see batch_share: 23 of 16 grids of 64 .. 192
     // nodes per axis, 10 where 128 nodes per level and CU leave the chains)
     gb.load = (int) std::min(64.0*perCU/800.0, 64.0);

@@ -169,3 +169,52 @@ def test_more_sweeps_than_the_record_has_numbers():
             tt, _oracle(vel, nz, nx, ny, D, SOURCE, nsweep))
         assert last is None or np.any(tt != last)
         last = tt
+
+
+@pytest.mark.parametrize("precision,nsweep,cube", [
+    (0, 36, True), (0, 7, False), (1, 5, True)])
+def test_chunked_batch_of_many_grids(precision, nsweep, cube):
+    """A batch large enough for the chunked tiles (24,576 nodes per level of
+    the longest sweep), of ragged grids and one whose field keeps changing:
+    every field equals the streamed tiles', some the oracle's too."""
+    rng = np.random.default_rng(71)
+    dims = [SERPENTINE] + [tuple(int(n) for n in rng.integers(30, 65, 3))
+                           for _ in range(80)]
+    nodes = sum(a * b * c for a, b, c in dims)
+    assert nodes >= 96 * 256 * max(map(sum, dims))
+    print("case: batch of many", precision, nsweep, cube, flush=True)
+    d = D if cube else (9.0, 10.0, 12.0)
+    models = [_serpentine(*SERPENTINE)]
+    models += [_model(*n, 400 + i) if i % 3 else np.repeat(
+        np.linspace(2000.0, 5000.0, n[2] - 1), (n[0] - 1) * (n[1] - 1))
+        for i, n in enumerate(dims[1:])]
+    srcs = [SOURCE] + [tuple(rng.uniform(0, n - 2.1) * h for n, h in
+                             zip(n, d)) for n in dims[1:]]
+    L, ierr = lib(), c_int(1)
+    L.fteik_batch3d_initialize(len(dims), byref(ierr))
+    assert ierr.value == 0
+    for i, n in enumerate(dims):
+        L.fteik_batch3d_setGrid(i + 1, *n, 0.0, 0.0, 0.0, *d, _d(models[i]),
+                                *srcs[i], byref(ierr))
+        assert ierr.value == 0
+    L.fteik_batch3d_setPrecision(precision, byref(ierr))
+    fields = []
+    for tile in (None, 12):
+        if tile is not None:
+            L.fteik_batch3d_setTile(tile, byref(ierr))
+            assert ierr.value == 0
+        L.fteik_batch3d_solve(nsweep, 3.0, byref(ierr))
+        # 2: corrections of a mixed solve that ran out before it converged
+        assert ierr.value in ((0, 2) if precision else (0,))
+        got = [np.zeros(a * b * c) for a, b, c in dims]
+        for i, tt in enumerate(got):
+            L.fteik_batch3d_getTravelTimeField64f(i + 1, tt.size, 0, _d(tt),
+                                                  byref(ierr))
+            assert ierr.value == 0
+        fields.append(got)
+    L.fteik_batch3d_free()
+    for a, b in zip(*fields):
+        np.testing.assert_array_equal(a, b)
+    for i in (0, 1, 2, 80) if precision == 0 else ():
+        np.testing.assert_array_equal(
+            fields[0][i], _oracle(models[i], *dims[i], d, srcs[i], nsweep))
