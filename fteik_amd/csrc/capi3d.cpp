@@ -418,8 +418,14 @@ void fteik_solver3d_initialize(int nz, int nx, int ny, double z0, double x0,
     // by tile: a solve of 33 x 29 x 31 nodes 2.2 -> 1.6 ms, 101^3 6.3 -> 5.1
     // ms, 257^3 104 -> 84 ms, 131 x 190 x 157 in mixed precision 60 -> 49 ms
     // (streamed tiles with tile skipping before).  The initialization sweeps
-    // keep the tile above.
-    g3.chunked = g3.chunkFits;
+    // keep the tile above.  Thin plates keep it in every sweep: a tile there
+    // is a few chunks, and a sweep with little to do is a mailbox exchange
+    // for every tile from corner to corner, where the streamed tiles' plan
+    // leaves the clean ones out (3 x 257 x 257 nodes, 12 iterations 33.9 ms,
+    // chunked 41.4; 9 x 257 x 257 in mixed precision 63.2 and 66.3; 17 x 513
+    // x 513, 8 iterations 65.2 and 63.7).
+    const int hops = (nx + 6)/8 + (ny + 6)/8 - 2;
+    g3.chunked = g3.chunkFits && !(nz < 16 && hops > 48);
     // sweep chains: the first mode-2 tile with two sweeps' tiles resident
     g3.ncu_chain = g_dev.ncu > 0 ? g_dev.ncu : 256;
     g3.overlapForced = false;

@@ -126,9 +126,9 @@ void fteik_solver3d_setMixedParameters(double bias, int maxCorrections,
  * rather than hanging.  Until a shape is chosen the shapes that getTile
  * reports serve the initialization sweeps, and the iterations run on chunked
  * 8 x 8 tiles, which skip nodes that cannot change (grids too large for
- * 32-bit offsets, or no memory for the change record: the reported shapes
- * serve every sweep).  autotune keeps the chunked tiles if they are faster
- * than every shape. */
+ * 32-bit offsets, wide plates of fewer than 16 levels, or no memory for the
+ * change record: the reported shapes serve every sweep).  autotune keeps the
+ * chunked tiles if they are faster than every shape. */
 void fteik_solver3d_setTile(int tile, int tile32, int *ierr);
 void fteik_solver3d_getTile(int *tile, int *tile32, int *ntiles, int *ierr);
 /* EXTENSION: the autotuner.  Solves source isrc (1-based) once with every
@@ -310,8 +310,9 @@ void fteik_batch3d_setMixedParameters(double bias, int maxCorrections,
 /* tile shape of the batch (see fteik_solver3d_setTile), flag (mode 0) or
  * mailbox (modes 1, 2); it serves every sweep.  Until one is chosen the
  * initialization sweeps run on mailbox tile 12 and the iterations on chunked
- * 8 x 8 tiles, which skip nodes that cannot change (grids too large for
- * 32-bit offsets, or no memory for their change record: tile 12) */
+ * 8 x 8 tiles, which skip nodes that cannot change (too few nodes to keep the
+ * GPU full of them, grids too large for 32-bit offsets, or no memory for
+ * their change record: tile 12) */
 void fteik_batch3d_setTile(int tile, int *ierr);
 /* EXTENSION: the batch autotuner: times fteik_batch3d_solve(nsweep, eps)
  * with every tile shape (flag and mailbox tiles), keeps the fastest and
