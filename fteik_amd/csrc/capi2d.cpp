@@ -287,7 +287,8 @@ static bool solve2d_range(int first, int n, const char *who)
         fteik_k_solve2d(fields, g2.d_slow, g2.nz, g2.nx, g2.dz, g2.dx, g2.eps,
                         0.0, 0.0, 0, 0, g2.nsweep, n, (int) ngrd, g2.d_sa,
                         g2.d_sa + n, g2.d_si, g2.d_si + n, g2.schedule,
-                        g2.d_err, g_dev.stream))
+                        g_dev.ncu > 0 ? g_dev.ncu : 256, g2.d_err,
+                        g_dev.stream))
         return false;
     {
         int e = 0;

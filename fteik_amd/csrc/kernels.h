@@ -213,7 +213,7 @@ int fteik_k_solve2d(double* tt, const double* slow, int nz, int nx,
                     int zsi, int xsi, int nsweep, int nsrc_batch,
                     int ld_tt, const double* zsa_v, const double* xsa_v,
                     const int* zsi_v, const int* xsi_v, int schedule,
-                    int* err, hipStream_t stream);
+                    int ncu, int* err, hipStream_t stream);
 
 // locate.hip
 int fteik_k_tables_d2f(float* tables, const double* tt, int ngrd,

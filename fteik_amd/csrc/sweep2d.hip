@@ -7,7 +7,8 @@
 // reference's bit for bit -- by one workgroup per source.  Two schedules:
 // solve2d_pipe_kernel (default) pipelines one column per lane without
 // barriers; solve2d_kernel (level by level, one barrier per level) is the
-// cross-check and serves grids wider than kMaxStrips strips of 64 columns.
+// cross-check, serves grids wider than kMaxStrips strips of 64 columns, and
+// many sources on wide grids of short columns.
 // Several sources (solveLSM) run as independent workgroups of one launch.
 #include <hip/hip_runtime.h>
 #include <type_traits>
@@ -521,14 +522,23 @@ extern "C" int fteik_k_solve2d(double* tt, const double* slow, int nz, int nx,
                                double xsa, int zsi, int xsi, int nsweep,
                                int nsrc_batch, int ld_tt, const double* zsa_v,
                                const double* xsa_v, const int* zsi_v,
-                               const int* xsi_v, int schedule, int* err,
-                               hipStream_t stream)
+                               const int* xsi_v, int schedule, int ncu,
+                               int* err, hipStream_t stream)
 {
     (void) zsa; (void) xsa; (void) zsi; (void) xsi;
     // pipelined columns while every strip has a counter and rows fit 24-bit
     // products
     const int strips = (nx - 1 + 63)/64;
-    if (schedule == 0 && strips <= kMaxStrips && nz < (1 << 23) && err) {
+    // Two workgroups of the level kernel fit a CU, one of the other.  With
+    // more sources than CUs on grids of several passes and short columns, of
+    // which a strip's 64 skewed columns do little at a time, the level kernel
+    // is the faster one: 1,024 sources of 5 x 577 nodes 8.7 ms against 11.5,
+    // 40 x 1,100 23.1 against 24.7, 80 x 1,100 28.4 against 26.2, 40 x 2,000
+    // 48.6 against 44.3.
+    const bool shortColumns = strips > T2P/64 && nsrc_batch > ncu &&
+                              nz < 125 - nx/19;
+    if (schedule == 0 && strips <= kMaxStrips && nz < (1 << 23) && err &&
+        !shortColumns) {
         const int threads = 64*(strips < T2P/64 ? strips : T2P/64);
         hipLaunchKernelGGL((solve2d_pipe_kernel<T2P>), dim3(nsrc_batch),
                            dim3(threads), 0, stream, tt, slow, nz, nx, dz, dx,

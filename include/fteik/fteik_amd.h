@@ -204,8 +204,9 @@ void fteik_solver2d_setSphereToCartEpsilon(double eps, int *ierr);
 void fteik_solver2d_setVerbosity(int verbose);
 void fteik_solver2d_setConvergenceTolerance(double convTol);
 /* EXTENSION: 0 = pipelined columns, one lane per x column walking down z,
- * no barrier per level (default; grids of more than 65,537 columns or
- * 2^23 rows run the level schedule); 1 = level by level with a workgroup barrier per
+ * no barrier per level (default; grids of more than 65,537 columns or 2^23
+ * rows, and more sources than CUs on wide grids of fewer than about 100 rows,
+ * run the level schedule); 1 = level by level with a workgroup barrier per
  * level (diagnostic).  Both give the same results bit for bit. */
 void fteik_solver2d_setSchedule(int schedule, int *ierr);
 /* solver2D.F90:283, :310: rays to the last solved source (as the 3D
