@@ -446,11 +446,35 @@ __device__ __forceinline__ double noinit2d(const Consts<double>& c, double tv,
                                            double s2, double s3)
 {
     double temtv = te - tv;
+    double t12min = rmin(tv + c.dz*s1, te + c.dx*s2);
+    double t1_2d = kHuge;
+    if (temtv < c.dz*s3 && -temtv < c.dx*s3) {
+        double sref2 = s3*s3;
+        double ta = tev + temtv;
+        double tb = tev - temtv;
+        double tab = ta - tb;
+        double tab2 = tab*tab;
+        double four_sref2 = 4.0*sref2;
+        t1_2d = ((tb*c.dz2i + ta*c.dx2i)
+              + __builtin_sqrt(four_sref2*c.dz2i_p_dx2i - c.dz2i_dx2i*tab2))
+              *c.dz2i_p_dx2i_inv;
+    }
+    return rmin(t12min, t1_2d);
+}
+
+// The same value without the branch around the operator: the pipelined
+// sweeps overlap its chain with the next steps' inputs.  (The level kernel,
+// with a barrier after every level, is 2 to 14 % slower with it.)
+__device__ __forceinline__ double noinit2d_flat(const Consts<double>& c,
+                                                double tv, double te,
+                                                double tev, double s1,
+                                                double s2, double s3)
+{
+    double temtv = te - tv;
     double t12min = lmin(tv + c.dz*s1, te + c.dx*s2);
-    // Without the branch around the operator: the pipelined sweeps overlap
-    // its chain with the next steps' inputs.  With the gate open the root's
-    // argument is at least 4 s3^2 min(1/dz^2, 1/dx^2) but for rounding, which
-    // at extreme aspect ratios can leave 0, or less, whose NaN never won.
+    // With the gate open the root's argument is at least 4 s3^2 min(1/dz^2,
+    // 1/dx^2) but for rounding, which at extreme aspect ratios can leave 0, or
+    // less, whose NaN never won.
     const bool gate = temtv < c.dz*s3 && -temtv < c.dx*s3;
     double sref2 = s3*s3;
     double ta = tev + temtv;

@@ -435,8 +435,8 @@ void solve2d_pipe_kernel(double* __restrict__ ttall,
                                                            : nz - L0 - k + fj,
                                                ix, P, te, tep, t, s1, s2, cA));
                     } else {
-                        const double u = lmin(t, noinit2d(c, P, te, tep, s1,
-                                                          s2, cA));
+                        const double u = lmin(t, noinit2d_flat(
+                            c, P, te, tep, s1, s2, cA));
                         P = in ? u : P;
                     }
                     tep = te;
@@ -533,10 +533,10 @@ extern "C" int fteik_k_solve2d(double* tt, const double* slow, int nz, int nx,
     // more sources than CUs on grids of several passes and short columns, of
     // which a strip's 64 skewed columns do little at a time, the level kernel
     // is the faster one: 1,024 sources of 5 x 577 nodes 8.7 ms against 11.5,
-    // 40 x 1,100 23.1 against 24.7, 80 x 1,100 28.4 against 26.2, 40 x 2,000
-    // 48.6 against 44.3.
+    // 40 x 1,100 22.8 against 24.7, 80 x 1,100 28.4 against 26.2, 20 x 2,000
+    // 41.4 against 43.0, 40 x 2,000 48.6 against 44.3.
     const bool shortColumns = strips > T2P/64 && nsrc_batch > ncu &&
-                              nz < 125 - nx/19;
+                              nz < 130 - nx/19;
     if (schedule == 0 && strips <= kMaxStrips && nz < (1 << 23) && err &&
         !shortColumns) {
         const int threads = 64*(strips < T2P/64 ? strips : T2P/64);

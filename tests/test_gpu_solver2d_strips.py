@@ -53,7 +53,7 @@ def test_strips_match_oracle(nz, nx):
     L.fteik_solver2d_free()
 
 
-@pytest.mark.parametrize("nz,nx", [(20, 600), (97, 520), (98, 520)])
+@pytest.mark.parametrize("nz,nx", [(20, 600), (102, 520), (103, 520)])
 def test_many_sources_on_wide_grids(nz, nx):
     """More sources than CUs on both sides of the line between the schedules:
     receiver times of every source equal the level schedule's, the last
