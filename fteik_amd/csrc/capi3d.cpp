@@ -223,6 +223,15 @@ bool prepare_source3d(int isrc, const char *who)
 
 } // namespace
 
+// (no solve is under way: a solve allocates before its first sweep)
+bool fteik_capi::solver3d_reclaim()
+{
+    const bool any = g3.d_stamp || g3.d_lastchg || g3.d_runs;
+    dfree(g3.d_stamp); dfree(g3.d_lastchg); dfree(g3.d_runs);
+    if (any) g3.chunkFits = g3.chunked = false;
+    return any;
+}
+
 bool fteik_capi::solver3d_view(Solver3DView *v)
 {
     if (!g3.init || !g3.haveModel) return false;
@@ -361,14 +370,13 @@ void fteik_solver3d_initialize(int nz, int nx, int ny, double z0, double x0,
     g3.chunkFits = fteik_k_chunk_fits(nz, nx, ny, g3.mbBytes) != 0;
     if (g3.chunkFits) {
         const size_t rw = fteik_k_run_words(nx, ny);
-        if (dalloc(&g3.d_stamp, fteik_k_stamp_bytes(ngrd)) &&
-            dalloc(&g3.d_lastchg, fteik_k_record_words()) &&
-            dalloc(&g3.d_runs, rw)) {
+        if (dalloc_spare(&g3.d_stamp, fteik_k_stamp_bytes(ngrd)) &&
+            dalloc_spare(&g3.d_lastchg, fteik_k_record_words()) &&
+            dalloc_spare(&g3.d_runs, rw)) {
             hipMemsetAsync(g3.d_runs, 0, rw*sizeof(unsigned long long),
                            g_dev.stream);
         } else {
-            hipGetLastError();
-            dfree(g3.d_stamp); dfree(g3.d_lastchg); dfree(g3.d_runs);
+            solver3d_reclaim();
             g3.chunkFits = false;
         }
     }
@@ -826,6 +834,14 @@ void fteik_solver3d_solveSourceLSM(int isrc, int *ierr)
         return;
     }
     const long ngrd = (long) g3.nz*g3.nx*g3.ny;
+    const long ncell = (long) (g3.nz - 1)*(g3.nx - 1)*(g3.ny - 1);
+    if (g3.precision != 0 &&
+        ((!g3.d_tt32 && !dalloc(&g3.d_tt32, ngrd)) ||
+         (!g3.d_slow32 && !dalloc(&g3.d_slow32, ncell)))) {
+        msg("%s: out of GPU memory (mixed precision)", who);
+        *ierr = 1;
+        return;
+    }
     hipEventRecord(g3.ev0, g_dev.stream);
     if (!prepare_source3d(isrc, who)) { *ierr = 1; return; }
     hipMemsetAsync(g3.d_err, 0, sizeof(int), g_dev.stream);
@@ -854,17 +870,9 @@ void fteik_solver3d_solveSourceLSM(int isrc, int *ierr)
     } else if (ok) {
         // mixed precision: FP32 Gauss-Seidel iterations from the FP64
         // initialization, then FP64 correction iterations to convergence.
-        const long ncell = (long) (g3.nz - 1)*(g3.nx - 1)*(g3.ny - 1);
-        if (!g3.d_tt32) {
-            ok = dalloc(&g3.d_tt32, ngrd) && dalloc(&g3.d_slow32, ncell);
-            if (!ok) msg("%s: out of GPU memory (mixed precision)", who);
-        }
-        if (ok) {
-            ok = fteik_k_d2f(g3.d_slow32, g3.d_slow, ncell, g_dev.stream) == 0
-              && fteik_k_d2f(g3.d_tt32, g3.d_tt, ngrd, g_dev.stream) == 0
-              && fteik_k_consts_to_float(g3.d_cst, g3.d_cst32,
-                                         g_dev.stream) == 0;
-        }
+        ok = fteik_k_d2f(g3.d_slow32, g3.d_slow, ncell, g_dev.stream) == 0
+          && fteik_k_d2f(g3.d_tt32, g3.d_tt, ngrd, g_dev.stream) == 0
+          && fteik_k_consts_to_float(g3.d_cst, g3.d_cst32, g_dev.stream) == 0;
         SweepLaunch L32 = launch3d(true);
         L32.zsi = s.zsi; L32.xsi = s.xsi; L32.ysi = s.ysi;
         if (chain_ok(true)) {

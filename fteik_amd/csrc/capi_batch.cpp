@@ -53,6 +53,7 @@ struct Batch3D {
     // one after another after the grids' words; count: sweeps recorded
     unsigned char *d_stamp = nullptr;
     size_t stampCap = 0;
+    bool busy = false;               // descriptors with its address come
     unsigned count = 0;
     bool cube = false;               // every grid has equal spacings
     int load = 0;                    // how full the sweeps keep the CUs
@@ -78,9 +79,14 @@ void free_batch()
     gb = Batch3D();
 }
 
-// Device descriptors and the workgroup order for the current tile shape.
-bool batch_prepare(const char *who)
+// Device descriptors and the workgroup order for the current tile shape;
+// record: with the chunked tiles' change record.
+bool prepare_with(const char *who, bool record)
 {
+    if (!record) {
+        dfree(gb.d_stamp);
+        gb.stampCap = 0;
+    }
     const int ng = (int) gb.g.size();
     std::vector<fteik::BatchGrid> desc((size_t) ng);
     std::vector<int> dims(3*(size_t) ng);
@@ -143,7 +149,7 @@ bool batch_prepare(const char *who)
         levels = std::max(levels, x.nz + x.nx + x.ny);
     }
     const double perCU = nodes/levels/(g_dev.ncu > 0 ? g_dev.ncu : 256);
-    gb.chunked = gb.chunk && edge && perCU >= 96.0;
+    gb.chunked = gb.chunk && edge && record && perCU >= 96.0;
     // (in 64ths of the chunks, see batch_share: 23 of 16 grids of 64 .. 192
     // nodes per axis, 10 where 128 nodes per level and CU leave the chains)
     gb.load = (int) std::min(64.0*perCU/800.0, 64.0);
@@ -162,12 +168,10 @@ bool batch_prepare(const char *who)
         if (bytes > gb.stampCap) {
             dfree(gb.d_stamp);
             gb.stampCap = 0;
-            if (dalloc(&gb.d_stamp, bytes)) {
+            if (dalloc_spare(&gb.d_stamp, bytes))
                 gb.stampCap = bytes;
-            } else {
-                hipGetLastError();
+            else
                 gb.chunked = false;
-            }
         }
     }
     if (!gb.chunked) {
@@ -275,6 +279,16 @@ bool batch_prepare(const char *who)
     return true;
 }
 
+// What the record leaves too little memory for comes before it.
+bool batch_prepare(const char *who)
+{
+    gb.busy = true;
+    const bool ok = prepare_with(who, true) ||
+                    (gb.chunked && prepare_with(who, false));
+    gb.busy = false;
+    return ok;
+}
+
 bool batch_sweep(int sweep, bool linit, bool fp32, bool track)
 {
     if (gb.mbTile >= 0) {
@@ -338,6 +352,16 @@ double batch_updates_iter()
 }
 
 } // namespace
+
+// (no solve is under way: a solve allocates before its first sweep)
+bool fteik_capi::batch_reclaim()
+{
+    if (!gb.d_stamp || gb.busy) return false;
+    dfree(gb.d_stamp);
+    gb.stampCap = 0;
+    gb.mapTile = -1;
+    return true;
+}
 
 extern "C" {
 

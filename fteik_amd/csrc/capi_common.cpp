@@ -57,6 +57,13 @@ bool device_ok(const char *who)
     return true;
 }
 
+bool reclaim_memory()
+{
+    const bool a = locator_reclaim(), b = solver3d_reclaim(),
+               c = batch_reclaim();
+    return a || b || c;
+}
+
 bool h2d(void *d, const void *h, size_t bytes)
 {
     if (hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, g_dev.stream)

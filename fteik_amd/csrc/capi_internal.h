@@ -39,12 +39,30 @@ extern Device g_dev;
 // false, with a message naming `who`, when no GPU is usable.
 bool device_ok(const char *who);
 
+// Memory that only makes later calls faster and can do without: the
+// locator's index and the solvers' change records.  Frees it; false: there
+// was none.
+bool reclaim_memory();
+bool locator_reclaim();
+bool solver3d_reclaim();
+bool batch_reclaim();
+
+// Device memory; of what was only kept for speed (dalloc_spare: not even
+// that, for memory of that kind).
 template <typename T>
-inline bool dalloc(T **p, size_t n)
+inline bool dalloc_spare(T **p, size_t n)
 {
     *p = nullptr;
     if (n == 0) n = 1;
-    return hipMalloc((void **) p, n*sizeof(T)) == hipSuccess;
+    if (hipMalloc((void **) p, n*sizeof(T)) == hipSuccess) return true;
+    (void) hipGetLastError();
+    *p = nullptr;
+    return false;
+}
+template <typename T>
+inline bool dalloc(T **p, size_t n)
+{
+    return dalloc_spare(p, n) || (reclaim_memory() && dalloc_spare(p, n));
 }
 
 template <typename T>

@@ -52,7 +52,7 @@ bool grow(T **p, size_t *cap, size_t n)
     if (n <= *cap) return true;
     dfree(*p);
     *cap = 0;
-    if (!dalloc(p, n)) { (void) hipGetLastError(); return false; }
+    if (!dalloc_spare(p, n)) return false;
     *cap = n;
     return true;
 }
@@ -63,7 +63,8 @@ bool grow(T **p, size_t *cap, size_t n)
 // nz points per column neighbouring columns have nearly the same times:
 // among the divisors p of ngrd, the mean |T[c + p] - T[c]| has local minima
 // at nz (against p - 1, p + 1) and at nz*nx (against steps of nz).
-bool find_shape(int *nz, int *nx, int *ny)
+// false: GPU error, or no memory.
+bool find_shape(int *nz, int *nx, int *ny, bool *memory)
 {
     const int n = gl.ngrd;
     if (g_model.nz > 0 && (long) g_model.nz*g_model.nx*g_model.ny == n) {
@@ -75,7 +76,9 @@ bool find_shape(int *nz, int *nx, int *ny)
         int *d_p = nullptr;
         float *d_d = nullptr;
         d.assign(p.size(), 0.0f);
-        bool ok = dalloc(&d_p, p.size()) && dalloc(&d_d, p.size()) &&
+        *memory = dalloc_spare(&d_p, p.size()) &&
+                  dalloc_spare(&d_d, p.size());
+        bool ok = *memory &&
                   h2d(d_p, p.data(), p.size()*sizeof(int)) &&
                   fteik_k_locate_strides(gl.d_tab, gl.ldgrd, gl.ntf, n, d_p,
                                          (int) p.size(), d_d,
@@ -131,7 +134,9 @@ bool find_shape(int *nz, int *nx, int *ny)
 bool build()
 {
     fteik::LocIndex &g = gi.g;
-    if (!find_shape(&g.nz, &g.nx, &g.ny)) return false;
+    bool memory = true;
+    gi.off = true;                   // until it is laid out
+    if (!find_shape(&g.nz, &g.nx, &g.ny, &memory)) return !memory;
     g.ntf = gl.ntf;
     g.nt = fteik_k_locate_index_nt(g.ntf);
     g.lz = 2; g.lx = 2; g.ly = 2;
@@ -145,7 +150,6 @@ bool build()
     const long nb = (long) g.nbz*g.nbx*g.nby;
     g.nb = (int) nb;
     g.ns = g.nsz*g.nsx*g.nsy;
-    gi.off = true;                   // until it is laid out
     // blocks mostly empty (a shape unlike the block's): not worth it
     if (nb*64 > 4L*gl.ngrd) return true;
     // a copy of the tables: within a quarter of the memory that is free
@@ -158,8 +162,8 @@ bool build()
         !grow(&g.srep, &gi.srepCap, nsr)) return true;
     g.h = g.rep + nr/2;
     g.sh = g.srep + nsr/2;
-    if ((!g.tmax && !dalloc(&g.tmax, 1)) ||
-        (!g.npair && !dalloc(&g.npair, fteik::kLocCounts))) return true;
+    if ((!g.tmax && !dalloc_spare(&g.tmax, 1)) ||
+        (!g.npair && !dalloc_spare(&g.npair, fteik::kLocCounts))) return true;
     unsigned tm = 0;
     if (hipMemsetAsync(g.tmax, 0, sizeof(unsigned), g_dev.stream)
             != hipSuccess ||
@@ -184,17 +188,16 @@ bool work_space(int n)
         const long c = std::max(ne, gi.evCap), f = std::max(tf, gi.evTf);
         free_events();
         // best, t0 and over adjoin: one copy brings them back
-        if (!dalloc(&gi.v.o8, (size_t) (c*f)) ||
-            !dalloc(&gi.v.w8, (size_t) (c*f)) ||
-            !dalloc(&gi.v.h8, (size_t) (c*f)) ||
-            !dalloc(&gi.v.row, (size_t) (3*c*f)) ||
-            !dalloc(&gi.v.xn, (size_t) c) || !dalloc(&gi.v.kap, (size_t) c) ||
-            !dalloc(&gi.v.mar, (size_t) c) ||
-            !dalloc(&gi.v.best, (size_t) (2*c)) ||
-            !dalloc(&gi.d_obs, (size_t) (c*f)) ||
-            !dalloc(&gi.d_wt, (size_t) (c*f)) ||
-            !dalloc(&gi.d_skip, (size_t) (c*f))) {
-            (void) hipGetLastError();
+        if (!dalloc_spare(&gi.v.o8, (size_t) (c*f)) ||
+            !dalloc_spare(&gi.v.w8, (size_t) (c*f)) ||
+            !dalloc_spare(&gi.v.h8, (size_t) (c*f)) ||
+            !dalloc_spare(&gi.v.row, (size_t) (3*c*f)) ||
+            !dalloc_spare(&gi.v.xn, (size_t) c) || !dalloc_spare(&gi.v.kap, (size_t) c) ||
+            !dalloc_spare(&gi.v.mar, (size_t) c) ||
+            !dalloc_spare(&gi.v.best, (size_t) (2*c)) ||
+            !dalloc_spare(&gi.d_obs, (size_t) (c*f)) ||
+            !dalloc_spare(&gi.d_wt, (size_t) (c*f)) ||
+            !dalloc_spare(&gi.d_skip, (size_t) (c*f))) {
             free_events();
             return false;
         }
@@ -211,10 +214,9 @@ bool work_space(int n)
     const long need = (long) g.ns*eb;
     if (need > gi.pairCap) {
         free_pairs();
-        if (!dalloc(&g.lbs, (size_t) need) ||
-            !dalloc(&g.pair, 2*(size_t) need) ||
-            !dalloc(&g.lbc, 64*(size_t) need)) {
-            (void) hipGetLastError();
+        if (!dalloc_spare(&g.lbs, (size_t) need) ||
+            !dalloc_spare(&g.pair, 2*(size_t) need) ||
+            !dalloc_spare(&g.lbc, 64*(size_t) need)) {
             free_pairs();
             return false;
         }
@@ -294,6 +296,16 @@ bool locator_tables_changed()
     gi.ready = gi.off = false;
     gi.searches = gi.pause = 0;
     return settle_origin_times();
+}
+
+bool locator_reclaim()
+{
+    const bool any = gi.permCap || gi.evCap || gi.pairCap;
+    if (!any) return false;
+    const int through = gi.through;
+    index_release();
+    gi.through = through;
+    return true;
 }
 
 void index_release()

@@ -18,6 +18,8 @@
 #include <type_traits>
 #include "kernels.h"
 
+namespace fteik_capi { bool reclaim_memory(); }   // capi_internal.h
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -1259,8 +1261,15 @@ int fteik_k_gemm_bf16(const void* A, long sam, long sak, const void* B,
         if (g_split) hipFree(g_split);
         g_split = nullptr;
         g_split_cap = 0;
-        if (hipMalloc((void**) &g_split, need*sizeof(float)) != hipSuccess)
-            return 1;
+        if (hipMalloc((void**) &g_split, need*sizeof(float)) != hipSuccess) {
+            (void) hipGetLastError();
+            if (!fteik_capi::reclaim_memory() ||
+                hipMalloc((void**) &g_split, need*sizeof(float))
+                    != hipSuccess) {
+                g_split = nullptr;
+                return 1;
+            }
+        }
         g_split_cap = need;
     }
     g.P = g_split;
