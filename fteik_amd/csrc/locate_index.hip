@@ -373,12 +373,14 @@ __device__ __forceinline__ float misfit(Picks row, float xn,
 }
 
 // Blocks of the groups that stay: one wave per group and 64 events, a lane
-// per block, the blocks' representatives and differences in registers.  Each (group, event) that stays is entered in a list with its
-// 64 blocks' bounds; the list holds every pair of the batch, so it cannot
-// overflow.
-template <int NT>
+// per block, the blocks' representatives and differences in registers.  Each
+// (group, event) that stays is entered in a list with its 64 blocks' bounds;
+// the list holds every pair of the batch, so it cannot overflow.
+// COUNT: and counts the blocks left (the registers that takes cost 4 % of a
+// search, so searches without a limit do without).
+template <int NT, bool COUNT>
 __global__ __launch_bounds__(64)
-void k_children(LocIndex g, fteik::LocEvents v, int e0, int n, unsigned limit)
+void k_children(LocIndex g, fteik::LocEvents v, int e0, int n)
 {
     // a group's waves adjoin: they read the same blocks, and its pairs adjoin
     // in the list
@@ -429,14 +431,14 @@ void k_children(LocIndex g, fteik::LocEvents v, int e0, int n, unsigned limit)
         const float lb = b >= 0 ? low_norm(ob, 2.0f*s2, v.kap[e], v.mar[e])
                                 : __builtin_inff();
         g.lbc[(long) at*64 + lane] = lb;
-        if (limit != ~0u) {
+        if (COUNT) {
             // (by the minimum at the wave's start: rather too many)
             const float kp = __uint_as_float((unsigned)
                 __builtin_amdgcn_readlane((int) __float_as_uint(keep), w));
             left += __popcll(__ballot(b >= 0 && stays(lb, kp)));
         }
     }
-    if (limit != ~0u && lane == 0)
+    if (COUNT && lane == 0)
         atomicAdd(g.npair + (1 + (blockIdx.x & 63))*kLocLine, left);
 }
 
@@ -579,8 +581,12 @@ int fteik_k_locate_index_search(const LocIndex* g, const fteik::LocEvents* v,
     const dim3 gc((unsigned) g->ns*(unsigned) ((n + 63)/64));
     // waves of k_cells: what the registers of NT times leave resident
 #define LI(N) case N: \
-        hipLaunchKernelGGL(k_children<N>, gc, dim3(64), 0, s, *g, *v, e0, n, \
-                           limit); \
+        if (limit == ~0u) \
+            hipLaunchKernelGGL((k_children<N, false>), gc, dim3(64), 0, s, \
+                               *g, *v, e0, n); \
+        else \
+            hipLaunchKernelGGL((k_children<N, true>), gc, dim3(64), 0, s, \
+                               *g, *v, e0, n); \
         hipLaunchKernelGGL(k_cells<N>, dim3((N <= 32 ? 32 : N <= 64 ? 20 : 16) \
                                             *((ncu + 7)/8*8)), \
                            dim3(64), 0, s, *g, *v, n <= 64 ? 8 : 1, limit, \
