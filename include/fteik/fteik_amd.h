@@ -162,7 +162,8 @@ void fteik_solver3d_setChainTile(int tile, int tile32, int *ierr);
 void fteik_solver3d_getSweepOverlap(int *on, int *tile, int *tile32,
                                     int *ierr);
 /* EXTENSION: device time of the last solve (ms, hipEvent), number of FP64
- * correction iterations run (mixed mode) and node updates performed. */
+ * correction iterations run (mixed mode) and node updates of the sweeps run
+ * (nodes that skipping left out count too). */
 void fteik_solver3d_getLastSolveInfo(double *ms, int *corrIterations,
                                      double *updates, int *ierr);
 
@@ -274,8 +275,15 @@ void locate_computeStatics32fF(const int *ldo, const int *nobs,
  * (locate.F90:122, :200-203).  0 gives every event a fresh origin-time
  * estimate and searches the grid points only. */
 void locate_setReferenceCompatibility(int mode, int *ierr);
-/* EXTENSION: locates events evnmbr[0..n-1] (1-based) in one pass over the
- * tables, each with a fresh origin-time estimate. */
+/* EXTENSION: locates events evnmbr[0..n-1] (1-based) together, each with a
+ * fresh origin-time estimate.  Calls of up to 8,192 events go through an index
+ * of the tables where that is faster: formed once per set of tables, it leaves
+ * out cells whose misfit provably exceeds one already found, so cells,
+ * objectives and origin times are those of the full search bit for bit.  It
+ * keeps a copy of the tables (within a quarter of the free memory) and up to
+ * 1 GB of work space until locate_finalize, or until a call runs out of
+ * memory.  Larger calls, tables or picks that are not finite, and picks that
+ * the index does not help make one pass over all tables' cells. */
 void locate_locateEvents(int n, const int *evnmbr, int *optIndx,
                          double *t0Opt, double *objOpt, int *ierr);
 /* EXTENSION (no counterpart in the reference): locate_locateEvents without
@@ -322,6 +330,7 @@ void fteik_batch3d_setTile(int tile, int *ierr);
  * shape of their initialization sweeps. */
 void fteik_batch3d_autotune(int nsweep, double eps, int *tile, int *ierr);
 void fteik_batch3d_solve(int nsweep, double eps, int *ierr);
+/* as fteik_solver3d_getLastSolveInfo */
 void fteik_batch3d_getLastSolveInfo(double *ms, int *corrIterations,
                                     double *updates, int *ierr);
 void fteik_batch3d_getTravelTimeField64f(int igrid, int ngrd, int order,
