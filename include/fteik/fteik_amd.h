@@ -273,7 +273,8 @@ void locate_computeStatics32fF(const int *ldo, const int *nobs,
  * (locate.F90:212, :687) and, for fewer than 512 grid points, the zero
  * padding of the objective array takes part in the minimum search
  * (locate.F90:122, :200-203).  0 gives every event a fresh origin-time
- * estimate and searches the grid points only. */
+ * estimate and searches the grid points only, through the same index as
+ * locate_locateEvents where that is faster; mode 1 passes over all cells. */
 void locate_setReferenceCompatibility(int mode, int *ierr);
 /* EXTENSION: locates events evnmbr[0..n-1] (1-based) together, each with a
  * fresh origin-time estimate.  Calls of up to 8,192 events go through an index
